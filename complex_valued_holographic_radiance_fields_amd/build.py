@@ -37,6 +37,7 @@ SOURCES = [
     "raster_render.hip",
     "asm_prop.hip",
     "asm_fft.hip",
+    "asm_any.hip",
     "hrf_capi.hip",
     "preprocess.hip",
     "optim.hip",

@@ -1,0 +1,1214 @@
+// asm_any.hip — the fused propagation passes of asm_fft.hip for the padded
+// lengths M without a compiled plan there: LDS transforms whose radices are
+// chosen at run time, for any multiple of four up to 4096.
+//
+// The passes and the intermediate layout are those of asm_fft.hip (rows in,
+// columns with the transfer function, rows out).  Without them such a grid
+// takes a zero pad, a library FFT of two passes and two transposes per
+// direction, a spectral multiply and a crop, about 12 trips of every M x M
+// grid through memory.  Both measured, forward / adjoint, by hipEvents:
+//
+//   fields            grid   library path         these passes
+//   1   (720 x 1280)  2560    229 /  215 us        96 /  92 us
+//   9   (300 x 400)    800    156 /  147 us        69 /  68 us
+//   18  (378 x 504)   1008    379 /  340 us       103 / 105 us
+//   9   (556 x 742)   1484   1195 / 1143 us       397 / 342 us   (chirp)
+//   3   (1424 x 1900) 3800   3000 / 2945 us       887 / 833 us   (chirp)
+//
+// The column passes are bound by VALU issue and the latency between their
+// barriers (1008 points, 18 fields: 72 us of the 103), the row passes by
+// memory latency.
+//
+// Smooth lengths (factors 2, 3, 5, 7): the forward transform is
+// decimated in frequency and leaves its output in digit-reversed order, the
+// inverse is decimated in time and takes that order.  Every butterfly then
+// writes back to the places it read, so a stage needs one barrier and holds
+// nothing across it, and no pass ever reorders: the column passes look the
+// frequency of a position up (the first digits from a table, the last digit
+// adds its multiple of M / R), and the row spectra stay in reversed order in
+// memory.  The last forward stage (span 1) hands its outputs to the transfer
+// function in registers, and the first inverse stage takes them from there.
+//
+// Other lengths: Bluestein's algorithm (the chirp transform; L. Bluestein,
+// 1970) on a smooth length L >= M + M/2 - 1: with c[n] = exp(-i pi n^2 / M),
+// X[k] = c[k] sum_n (x[n] c[n]) conj(c)[k - n], a convolution by a forward
+// transform of L points, a product with the chirp's spectrum (made in double
+// on the host, in digit-reversed order) in registers, and an inverse
+// transform.  The factors c[k] on the spectrum side cancel between a forward
+// and the following inverse transform (|c| = 1) in both directions, so only
+// field samples are ever multiplied by the chirp.  A field occupies at most
+// M/2 samples of the line, [M/4, 3M/4), and as many are kept, hence
+// L >= 3M/2 - 1 and not 2M - 1.
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+#include <complex>
+#include <map>
+#include <mutex>
+#include <vector>
+
+#include "asm_common.h"
+#include "fast_trig.h"
+#include "fft_dft.h"
+#include "hrf_internal.h"
+
+namespace hrf {
+namespace {
+
+constexpr int kAnyMaxStages = 6;
+constexpr int kAnyMinM = 32;
+constexpr int kAnyMaxM = 4096;
+// The outer radix of the chirp transforms.  Its butterfly owns positions
+// j + t L/16: the M <= (L + 1) / 1.5 spectrum entries are at t < 11, the M/2
+// field samples at t < 6.
+constexpr int kChirpOuter = 16, kChirpSpec = 11, kChirpField = 6;
+
+struct AnyStage {
+  int radix;
+  int span;    // D: distance between a butterfly's inputs
+  int tw;      // offset of the stage's twiddles
+  float inv;   // 1 / D
+};
+
+// A transform length's stages in forward order (spans decreasing to 1).
+struct AnyPlan {
+  int n;
+  int stages;
+  AnyStage st[kAnyMaxStages];
+};
+
+// LDS layout: transform b of the batch starts at b * line_stride; a half
+// wave's lanes then hold eight consecutive elements of four transforms (16
+// of two) on different banks wherever the span is at least eight.
+template <int B>
+__host__ __device__ constexpr int line_stride(int n) {
+  constexpr int want = B == 4 ? 8 : 16;  // modulo 32 elements (256 bytes)
+  return n + ((want - n % 32) + 32) % 32;
+}
+
+// ---------------------------------------------------------------- stages --
+// The thread index through an empty asm: a stage inside the plane loop of a
+// column pass then computes its addresses there, instead of the compiler
+// holding those of every radix case in registers through the loop.  With the
+// stores' addresses formed again (mid_stage) and no radix above 16's register
+// need, the column passes spill at most 21 registers at 128, from 60-80: 136
+// -> 72 us (1008 points, 18 fields), 110 -> 62 us (2560 points, one).  Radices
+// 11 and 13 are left out for that: their lengths take the chirp transform.
+__device__ __forceinline__ unsigned opaque_tid() {
+  unsigned tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  return tid;
+}
+
+// j / D for j < 2^13, D < 2^12: (j + 1/2) / D is at least 1 / 2D away from an
+// integer, and the float quotient is off by less than that.
+__device__ __forceinline__ unsigned quotient(unsigned j, float inv) {
+  return static_cast<unsigned>((static_cast<float>(j) + 0.5f) * inv);
+}
+
+// Stage with both its sides in LDS.  DIT: inverse transform (conjugate
+// twiddles before the butterfly), else forward (twiddles after it).
+template <int R, int B, bool DIT>
+__device__ __forceinline__ void mid_stage(float2* lds, int ld, unsigned D, float inv, int n,
+                                          const float2* __restrict__ w) {
+  const unsigned nb = B * (n / R);
+  for (unsigned q = opaque_tid(); q < nb; q += blockDim.x) {
+    const unsigned j = q / B, b = q % B;
+    const unsigned hi = quotient(j, inv), lo = j - hi * D;
+    unsigned a = b * ld + hi * (D * R) + lo;
+    float2 x[R];
+#pragma unroll
+    for (int t = 0; t < R; ++t) x[t] = lds[a + t * D];
+    if (DIT) {
+#pragma unroll
+      for (int t = 1; t < R; ++t) {
+        const float2 v = w[(t - 1) * D + lo];
+        x[t] = cmulf(x[t], make_float2(v.x, -v.y));
+      }
+    }
+    Dft<R, DIT>::run(x);
+    if (!DIT) {
+#pragma unroll
+      for (int t = 1; t < R; ++t) x[t] = cmulf(x[t], w[(t - 1) * D + lo]);
+    }
+    // The addresses are formed again for the stores, not held meanwhile.
+    asm volatile("" : "+v"(a));
+#pragma unroll
+    for (int t = 0; t < R; ++t) lds[a + t * D] = x[t];
+  }
+}
+
+// First forward stage: inputs from in(position, transform, t), of which only
+// those at t < NT can be nonzero.  ONCE: the block has a thread for every
+// butterfly (the caller's per-thread arrays are indexed by t).
+template <int R, int B, int NT, bool ONCE, class In>
+__device__ __forceinline__ void first_stage(float2* lds, int ld, unsigned D,
+                                            const float2* __restrict__ w, In& in) {
+  for (unsigned q = opaque_tid(); q < B * D; q += ONCE ? ~0u / 2 : blockDim.x) {
+    const unsigned j = q / B, b = q % B;
+    float2 x[R];
+#pragma unroll
+    for (int t = 0; t < R; ++t)
+      x[t] = t < NT ? in(static_cast<int>(j + t * D), static_cast<int>(b), t)
+                    : make_float2(0.0f, 0.0f);
+    Dft<R, false>::run(x);
+    float2* p = lds + (b * ld + j);
+    p[0] = x[0];
+#pragma unroll
+    for (int t = 1; t < R; ++t) p[t * D] = cmulf(x[t], w[(t - 1) * D + j]);
+  }
+}
+
+// Last inverse stage: outputs to out(position, transform, t, value), those at
+// t < NT only.
+template <int R, int B, int NT, bool ONCE, class Out>
+__device__ __forceinline__ void last_stage(const float2* lds, int ld, unsigned D,
+                                           const float2* __restrict__ w, Out& out) {
+  for (unsigned q = opaque_tid(); q < B * D; q += ONCE ? ~0u / 2 : blockDim.x) {
+    const unsigned j = q / B, b = q % B;
+    const float2* p = lds + (b * ld + j);
+    float2 x[R];
+    x[0] = p[0];
+#pragma unroll
+    for (int t = 1; t < R; ++t) {
+      const float2 v = w[(t - 1) * D + j];
+      x[t] = cmulf(p[t * D], make_float2(v.x, -v.y));
+    }
+    Dft<R, true>::run(x);
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+      out(static_cast<int>(j + t * D), static_cast<int>(b), t, x[t]);
+  }
+}
+
+#define HRF_ANY_RADICES(X) X(3) X(4) X(5) X(6) X(7) X(8) X(9) X(10) X(12) X(16)
+
+// Middle stages first .. last - 1 in forward order, or the same backwards;
+// each starts with the barrier that publishes what it reads.
+template <int B, bool DIT>
+__device__ __forceinline__ void mid_stages(float2* lds, int ld, const AnyPlan* __restrict__ pl,
+                                           const float2* __restrict__ tw) {
+  const int n = pl->n, cnt = pl->stages - 2;
+  for (int i = 0; i < cnt; ++i) {
+    const int k = DIT ? cnt - i : 1 + i;
+    const unsigned D = pl->st[k].span;
+    const float inv = pl->st[k].inv;
+    const float2* w = tw + pl->st[k].tw;
+    __syncthreads();
+    switch (pl->st[k].radix) {
+#define HRF_ANY_CASE(R)                            \
+  case R:                                          \
+    mid_stage<R, B, DIT>(lds, ld, D, inv, n, w);   \
+    break;
+      HRF_ANY_RADICES(HRF_ANY_CASE)
+#undef HRF_ANY_CASE
+      default:
+        break;
+    }
+  }
+}
+template <int B, class In>
+__device__ __forceinline__ void first_stage_any(float2* lds, int ld,
+                                                const AnyPlan* __restrict__ pl,
+                                                const float2* __restrict__ tw, In& in) {
+  const unsigned D = pl->st[0].span;
+  switch (pl->st[0].radix) {
+#define HRF_ANY_CASE(R)                            \
+  case R:                                          \
+    first_stage<R, B, R, false>(lds, ld, D, tw, in); \
+    break;
+    HRF_ANY_RADICES(HRF_ANY_CASE)
+#undef HRF_ANY_CASE
+    default:
+      break;
+  }
+}
+template <int B, class Out>
+__device__ __forceinline__ void last_stage_any(const float2* lds, int ld,
+                                               const AnyPlan* __restrict__ pl,
+                                               const float2* __restrict__ tw, Out& out) {
+  const unsigned D = pl->st[0].span;
+  switch (pl->st[0].radix) {
+#define HRF_ANY_CASE(R)                            \
+  case R:                                          \
+    last_stage<R, B, R, false>(lds, ld, D, tw, out); \
+    break;
+    HRF_ANY_RADICES(HRF_ANY_CASE)
+#undef HRF_ANY_CASE
+    default:
+      break;
+  }
+}
+
+// The R contiguous elements of a span-1 butterfly (16-byte accesses: the
+// line stride and R are even).
+template <int R>
+__device__ __forceinline__ void load_inner(const float2* p, float2 (&x)[R]) {
+  if constexpr (R % 2 == 0) {
+#pragma unroll
+    for (int t = 0; t < R; t += 2) {
+      const float4 v = *reinterpret_cast<const float4*>(p + t);
+      x[t] = make_float2(v.x, v.y);
+      x[t + 1] = make_float2(v.z, v.w);
+    }
+  } else {
+#pragma unroll
+    for (int t = 0; t < R; ++t) x[t] = p[t];
+  }
+}
+template <int R>
+__device__ __forceinline__ void store_inner(float2* p, const float2 (&x)[R]) {
+  if constexpr (R % 2 == 0) {
+#pragma unroll
+    for (int t = 0; t < R; t += 2)
+      *reinterpret_cast<float4*>(p + t) = make_float4(x[t].x, x[t].y, x[t + 1].x, x[t + 1].y);
+  } else {
+#pragma unroll
+    for (int t = 0; t < R; ++t) p[t] = x[t];
+  }
+}
+
+// The chirp transform's innermost forward stage, the product with the
+// chirp's spectrum and the first inverse stage, in place (span 1).
+template <int R, int B, bool CONJ>
+__device__ __forceinline__ void conv_stage(float2* lds, int ld, int n,
+                                           const float2* __restrict__ spec) {
+  const unsigned nb = B * (n / R);
+  for (unsigned q = opaque_tid(); q < nb; q += blockDim.x) {
+    const unsigned j = q / B, b = q % B;
+    float2* p = lds + (b * ld + j * R);
+    float2 x[R];
+    load_inner<R>(p, x);
+    Dft<R, false>::run(x);
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      const float2 v = spec[j * R + t];
+      x[t] = cmulf(x[t], make_float2(v.x, CONJ ? -v.y : v.y));
+    }
+    Dft<R, true>::run(x);
+    store_inner<R>(p, x);
+  }
+}
+
+// Everything between the chirp transform's first and last stage.
+template <int B, bool CONJ>
+__device__ __forceinline__ void chirp_middle(float2* lds, int ld, const AnyPlan* __restrict__ pl,
+                                             const float2* __restrict__ tw,
+                                             const float2* __restrict__ spec) {
+  const int n = pl->n;
+  mid_stages<B, false>(lds, ld, pl, tw);
+  __syncthreads();
+  switch (pl->st[pl->stages - 1].radix) {
+#define HRF_ANY_CASE(R)                            \
+  case R:                                          \
+    conv_stage<R, B, CONJ>(lds, ld, n, spec);      \
+    break;
+    HRF_ANY_CASE(3)
+    HRF_ANY_CASE(4)
+    HRF_ANY_CASE(5)
+    HRF_ANY_CASE(7)
+    HRF_ANY_CASE(9)
+#undef HRF_ANY_CASE
+    default:
+      break;
+  }
+  mid_stages<B, true>(lds, ld, pl, tw);
+  __syncthreads();
+}
+
+// What a pass needs of a padded length, in device memory.
+struct AnyTab {
+  const AnyPlan* plan;
+  const float2* tw;
+  const uint16_t* freq;   // smooth: frequency of position j * (last radix)
+  const float2* chirp;    // chirp: c[M/4 + i], i < M/2
+  const float2* spec;     // chirp: spectrum of conj(c), digit-reversed, / L
+  int M;                  // padded length
+  int n;                  // transform length (M, or L)
+  int outer;              // n / (first radix)
+  int inner;              // last radix
+};
+
+extern __shared__ __align__(16) float2 any_lds[];
+
+// ------------------------------------------------------------ row passes --
+// As k_rows_in / k_rows_out of asm_fft.hip.  The spectrum side of a smooth
+// length is in digit-reversed order: its last forward stage (radix 4, 8, 12
+// or 16, span 1) gives a thread whole rows of an intermediate tile.
+template <int R, int B>
+__device__ __forceinline__ void rows_store(const float2* lds, int ld, int M, float2* dst, int img,
+                                           int h, int r0) {
+  const unsigned nb = B * (M / R);
+  const int ncb = M / kFftBatch;
+  for (unsigned q = opaque_tid(); q < nb; q += blockDim.x) {
+    const unsigned j = q / B, b = q % B;
+    const int r = r0 + static_cast<int>(b);
+    if (r >= h) continue;
+    float2 x[R];
+    load_inner<R>(lds + (b * ld + j * R), x);
+    Dft<R, false>::run(x);
+#pragma unroll
+    for (int t = 0; t < R; t += 4) {
+      float4* o = reinterpret_cast<float4*>(
+          dst + tile_off(img, ncb, static_cast<int>(j * R + t) / 4, h, r, 0, 4));
+      o[0] = make_float4(x[t].x, x[t].y, x[t + 1].x, x[t + 1].y);
+      o[1] = make_float4(x[t + 2].x, x[t + 2].y, x[t + 3].x, x[t + 3].y);
+    }
+  }
+}
+template <int R, int B>
+__device__ __forceinline__ void rows_load(float2* lds, int ld, int M, const float2* src, int img,
+                                          int h, int r0) {
+  const unsigned nb = B * (M / R);
+  const int ncb = M / kFftBatch;
+  for (unsigned q = opaque_tid(); q < nb; q += blockDim.x) {
+    const unsigned j = q / B, b = q % B;
+    const int r = r0 + static_cast<int>(b);
+    float2 x[R];
+#pragma unroll
+    for (int t = 0; t < R; t += 4) {
+      float4 v0 = make_float4(0.0f, 0.0f, 0.0f, 0.0f), v1 = v0;
+      if (r < h) {
+        const float4* i = reinterpret_cast<const float4*>(
+            src + tile_off(img, ncb, static_cast<int>(j * R + t) / 4, h, r, 0, 4));
+        v0 = i[0];
+        v1 = i[1];
+      }
+      x[t] = make_float2(v0.x, v0.y);
+      x[t + 1] = make_float2(v0.z, v0.w);
+      x[t + 2] = make_float2(v1.x, v1.y);
+      x[t + 3] = make_float2(v1.z, v1.w);
+    }
+    Dft<R, true>::run(x);
+    store_inner<R>(lds + (b * ld + j * R), x);
+  }
+}
+
+template <int B>
+__global__ __launch_bounds__(512, 4) void k_any_rows_in(const float2* __restrict__ src,
+                                                     float2* __restrict__ dst, int h, int w_in,
+                                                     int c_in, AnyTab tab) {
+  float2* lds = any_lds;
+  const int ld = line_stride<B>(tab.n);
+  const int per = (h + B - 1) / B;
+  const int img = blockIdx.x / per, r0 = (blockIdx.x - img * per) * B;
+  const float2* srow = src + static_cast<int64_t>(img) * h * w_in;
+  auto in = [&](int pos, int rr, int) -> float2 {
+    const unsigned col = static_cast<unsigned>(pos - c_in);
+    const int r = r0 + rr;
+    return (r < h && col < static_cast<unsigned>(w_in))
+               ? srow[static_cast<int64_t>(r) * w_in + col]
+               : make_float2(0.0f, 0.0f);
+  };
+  first_stage_any<B>(lds, ld, tab.plan, tab.tw, in);
+  mid_stages<B, false>(lds, ld, tab.plan, tab.tw);
+  __syncthreads();
+  switch (tab.inner) {
+    case 16: rows_store<16, B>(lds, ld, tab.M, dst, img, h, r0); break;
+    case 12: rows_store<12, B>(lds, ld, tab.M, dst, img, h, r0); break;
+    case 8: rows_store<8, B>(lds, ld, tab.M, dst, img, h, r0); break;
+    default: rows_store<4, B>(lds, ld, tab.M, dst, img, h, r0); break;
+  }
+}
+
+template <int B>
+__global__ __launch_bounds__(512, 4) void k_any_rows_out(const float2* __restrict__ src,
+                                                      float2* __restrict__ dst, int h, int w_out,
+                                                      int c_out, float scale, AnyTab tab) {
+  float2* lds = any_lds;
+  const int ld = line_stride<B>(tab.n);
+  const int per = (h + B - 1) / B;
+  const int img = blockIdx.x / per, r0 = (blockIdx.x - img * per) * B;
+  switch (tab.inner) {
+    case 16: rows_load<16, B>(lds, ld, tab.M, src, img, h, r0); break;
+    case 12: rows_load<12, B>(lds, ld, tab.M, src, img, h, r0); break;
+    case 8: rows_load<8, B>(lds, ld, tab.M, src, img, h, r0); break;
+    default: rows_load<4, B>(lds, ld, tab.M, src, img, h, r0); break;
+  }
+  mid_stages<B, true>(lds, ld, tab.plan, tab.tw);
+  __syncthreads();
+  float2* drow = dst + static_cast<int64_t>(img) * h * w_out;
+  auto out = [&](int pos, int rr, int, float2 v) {
+    const unsigned i = static_cast<unsigned>(pos - c_out);
+    const int r = r0 + rr;
+    if (i < static_cast<unsigned>(w_out) && r < h)
+      drow[static_cast<int64_t>(r) * w_out + i] = cscale(v, scale);
+  };
+  last_stage_any<B>(lds, ld, tab.plan, tab.tw, out);
+}
+
+// Chirp versions: the spectrum side in natural order.
+template <int B>
+__global__ __launch_bounds__(768, 4) void k_chirp_rows_in(const float2* __restrict__ src,
+                                                       float2* __restrict__ dst, int h, int w_in,
+                                                       int c_in, AnyTab tab) {
+  float2* lds = any_lds;
+  const int ld = line_stride<B>(tab.n);
+  const int per = (h + B - 1) / B;
+  const int img = blockIdx.x / per, r0 = (blockIdx.x - img * per) * B;
+  const float2* srow = src + static_cast<int64_t>(img) * h * w_in;
+  const int shift = tab.M / 4 - c_in, ncb = tab.M / kFftBatch;
+  auto in = [&](int pos, int rr, int) -> float2 {
+    const unsigned col = static_cast<unsigned>(pos + shift);
+    const int r = r0 + rr;
+    return (r < h && col < static_cast<unsigned>(w_in))
+               ? cmulf(srow[static_cast<int64_t>(r) * w_in + col], tab.chirp[pos])
+               : make_float2(0.0f, 0.0f);
+  };
+  auto out = [&](int pos, int rr, int, float2 v) {
+    const int r = r0 + rr;
+    if (pos < tab.M && r < h) dst[tile_off(img, ncb, pos / 4, h, r, pos % 4, 4)] = v;
+  };
+  first_stage<kChirpOuter, B, kChirpField, false>(lds, ld, tab.outer, tab.tw, in);
+  chirp_middle<B, false>(lds, ld, tab.plan, tab.tw, tab.spec);
+  last_stage<kChirpOuter, B, kChirpSpec, false>(lds, ld, tab.outer, tab.tw, out);
+}
+
+template <int B>
+__global__ __launch_bounds__(768, 4) void k_chirp_rows_out(const float2* __restrict__ src,
+                                                        float2* __restrict__ dst, int h,
+                                                        int w_out, int c_out, float scale,
+                                                        AnyTab tab) {
+  float2* lds = any_lds;
+  const int ld = line_stride<B>(tab.n);
+  const int per = (h + B - 1) / B;
+  const int img = blockIdx.x / per, r0 = (blockIdx.x - img * per) * B;
+  const int shift = tab.M / 4 - c_out, ncb = tab.M / kFftBatch;
+  auto in = [&](int pos, int rr, int) -> float2 {
+    const int r = r0 + rr;
+    return (pos < tab.M && r < h) ? src[tile_off(img, ncb, pos / 4, h, r, pos % 4, 4)]
+                                  : make_float2(0.0f, 0.0f);
+  };
+  float2* drow = dst + static_cast<int64_t>(img) * h * w_out;
+  auto out = [&](int pos, int rr, int, float2 v) {
+    const unsigned i = static_cast<unsigned>(pos + shift);
+    const int r = r0 + rr;
+    if (i < static_cast<unsigned>(w_out) && r < h) {
+      const float2 c = tab.chirp[pos];
+      drow[static_cast<int64_t>(r) * w_out + i] =
+          cscale(cmulf(v, make_float2(c.x, -c.y)), scale);
+    }
+  };
+  first_stage<kChirpOuter, B, kChirpSpec, false>(lds, ld, tab.outer, tab.tw, in);
+  chirp_middle<B, true>(lds, ld, tab.plan, tab.tw, tab.spec);
+  last_stage<kChirpOuter, B, kChirpField, false>(lds, ld, tab.outer, tab.tw, out);
+}
+
+// --------------------------------------------------------- column passes --
+// kz of spectral element (row frequency i, column frequency k), -1 where the
+// evanescent cut or the aperture zeroes the transfer function.
+__device__ __forceinline__ float kz_or_cut(float k0, int i, int k, int M, float sfreq, float ap) {
+  float fx, fy;
+  bool inap, prop;
+  coords(i, k, M, sfreq, ap, &fx, &fy, &inap);
+  const float kk = kz_of(k0, fx, fy, &prop);
+  return prop && inap ? kk : -1.0f;
+}
+
+struct Band {
+  float fxm, fym, d;
+  bool all;
+};
+__device__ __forceinline__ Band band_of(const AsmFftConsts& mc, int p, int c) {
+  return Band{mc.fxmax[p * kMaxChannels + c], mc.fymax[p * kMaxChannels + c], mc.d[p],
+              mc.band_all[p * kMaxChannels + c] != 0};
+}
+// Whether the transfer function passes (i, k), given its kz.
+__device__ __forceinline__ bool passes(const Band& bd, float kz, int i, int k, int M,
+                                       float sfreq) {
+  if (kz < 0.0f) return false;
+  if (bd.all) return true;
+  float fx, fy;
+  bool inap;
+  coords(i, k, M, sfreq, -1.0f, &fx, &fy, &inap);
+  return fabsf(fx) < bd.fxm && fabsf(fy) < bd.fym;
+}
+__device__ __forceinline__ float2 turn(float2 x, float phase) {
+  float sn, cs;
+  sincos_big_ff(phase, &sn, &cs);
+  return make_float2(x.x * cs - x.y * sn, x.x * sn + x.y * cs);
+}
+
+// The block's channel, intermediate tile, first column in it and first
+// spectrum column.
+template <int B>
+__device__ __forceinline__ void column_block(int M, int* c, int* cb, int* col0, int* k0) {
+  int hb;
+  map_cblock(blockIdx.x, gridDim.x, c, &hb, M / B);
+  *cb = hb / (kFftBatch / B);
+  *col0 = (hb % (kFftBatch / B)) * B;
+  *k0 = hb * B;
+}
+
+// As k_col_fwd of asm_fft.hip.  A thread's U butterflies of the innermost
+// stage (radix R) own U R spectrum elements through the plane loop.
+template <int R, int U, int B>
+__global__ __launch_bounds__(R == 12 ? 704 : 512, 4) void k_any_col_fwd(const float2* __restrict__ X,
+                                                     float2* __restrict__ Z, int P, int C, int H,
+                                                     int r_pad, int S, int s_crop, float sfreq,
+                                                     float ap, AsmFftConsts mc, AnyTab tab,
+                                                     int accumulate) {
+  float2* lds = any_lds;
+  const int M = tab.M, ld = line_stride<B>(M), ncb = M / kFftBatch;
+  int c, cb, col0, k0;
+  column_block<B>(M, &c, &cb, &col0, &k0);
+  const float2* src = nullptr;
+  auto in = [&](int pos, int b, int) -> float2 {
+    const unsigned r = static_cast<unsigned>(pos - r_pad);
+    return r < static_cast<unsigned>(H) ? src[r * kFftBatch + b] : make_float2(0.0f, 0.0f);
+  };
+  const int T = static_cast<int>(blockDim.x), nb = B * (M / R);
+  const int b = threadIdx.x % B;
+  // Frequency of column k0 + b: position k0 + b is digit (k0 + b) % R of a
+  // butterfly.
+  const int kcol = tab.freq[(k0 + b) / R] + (k0 + b) % R * (M / R);
+  int fb[U];
+  float kz[U][R];
+  float2 acc[U][R];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int q = threadIdx.x + u * T;
+    fb[u] = q < nb ? tab.freq[q / B] : 0;
+#pragma unroll
+    for (int t = 0; t < R; ++t) {
+      acc[u][t] = make_float2(0.0f, 0.0f);
+      kz[u][t] = q < nb ? kz_or_cut(mc.k[c], fb[u] + t * (M / R), kcol, M, sfreq, ap) : -1.0f;
+    }
+  }
+  for (int p = 0; p < P; ++p) {
+    __syncthreads();
+    src = X + tile_off(p * C + c, ncb, cb, H, 0, 0, kFftBatch) + col0;
+    first_stage_any<B>(lds, ld, tab.plan, tab.tw, in);
+    mid_stages<B, false>(lds, ld, tab.plan, tab.tw);
+    __syncthreads();
+    const Band bd = band_of(mc, p, c);
+    const int tid = static_cast<int>(opaque_tid());
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = tid + u * T;
+      if (q < nb) {
+        asm volatile("" : "+v"(fb[u]));  // band-limit coordinates formed here
+        float2 x[R];
+        load_inner<R>(lds + (b * ld + q / B * R), x);
+        Dft<R, false>::run(x);
+#pragma unroll
+        for (int t = 0; t < R; ++t)
+          if (passes(bd, kz[u][t], fb[u] + t * (M / R), kcol, M, sfreq))
+            acc[u][t] = cadd(acc[u][t], turn(x[t], bd.d * kz[u][t]));
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int q = threadIdx.x + u * T;
+    if (q < nb) {
+      Dft<R, true>::run(acc[u]);
+      store_inner<R>(lds + (b * ld + q / B * R), acc[u]);
+    }
+  }
+  mid_stages<B, true>(lds, ld, tab.plan, tab.tw);
+  __syncthreads();
+  float2* dst = Z + tile_off(c, ncb, cb, S, 0, 0, kFftBatch) + col0;
+  auto out = [&](int pos, int bb, int, float2 v) {
+    const unsigned r = static_cast<unsigned>(pos - s_crop);
+    if (r < static_cast<unsigned>(S)) {
+      float2* o = dst + r * kFftBatch + bb;
+      *o = accumulate ? cadd(*o, v) : v;
+    }
+  };
+  last_stage_any<B>(lds, ld, tab.plan, tab.tw, out);
+}
+
+// As k_col_adj of asm_fft.hip.
+template <int R, int U, int B>
+__global__ __launch_bounds__(R == 12 ? 704 : 512, 4) void k_any_col_adj(const float2* __restrict__ X,
+                                                     float2* __restrict__ Z, int P, int C, int S,
+                                                     int s_pad, int H, int r_crop, float sfreq,
+                                                     float ap, AsmFftConsts mc, AnyTab tab) {
+  float2* lds = any_lds;
+  const int M = tab.M, ld = line_stride<B>(M), ncb = M / kFftBatch;
+  int c, cb, col0, k0;
+  column_block<B>(M, &c, &cb, &col0, &k0);
+  const float2* src = X + tile_off(c, ncb, cb, S, 0, 0, kFftBatch) + col0;
+  auto in = [&](int pos, int b, int) -> float2 {
+    const unsigned r = static_cast<unsigned>(pos - s_pad);
+    return r < static_cast<unsigned>(S) ? src[r * kFftBatch + b] : make_float2(0.0f, 0.0f);
+  };
+  const int T = static_cast<int>(blockDim.x), nb = B * (M / R);
+  const int b = threadIdx.x % B;
+  first_stage_any<B>(lds, ld, tab.plan, tab.tw, in);
+  const int kcol = tab.freq[(k0 + b) / R] + (k0 + b) % R * (M / R);
+  int fb[U];
+  float kz[U][R];
+  float2 g[U][R];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int q = threadIdx.x + u * T;
+    fb[u] = q < nb ? tab.freq[q / B] : 0;
+#pragma unroll
+    for (int t = 0; t < R; ++t)
+      kz[u][t] = q < nb ? kz_or_cut(mc.k[c], fb[u] + t * (M / R), kcol, M, sfreq, ap) : -1.0f;
+  }
+  mid_stages<B, false>(lds, ld, tab.plan, tab.tw);
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < U; ++u) {
+    const int q = threadIdx.x + u * T;
+    if (q < nb) {
+      load_inner<R>(lds + (b * ld + q / B * R), g[u]);
+      Dft<R, false>::run(g[u]);
+    }
+  }
+  for (int p = 0; p < P; ++p) {
+    __syncthreads();
+    const Band bd = band_of(mc, p, c);
+    const int tid = static_cast<int>(opaque_tid());
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int q = tid + u * T;
+      if (q < nb) {
+        asm volatile("" : "+v"(fb[u]));  // band-limit coordinates formed here
+        float2 x[R];
+#pragma unroll
+        for (int t = 0; t < R; ++t)
+          x[t] = passes(bd, kz[u][t], fb[u] + t * (M / R), kcol, M, sfreq)
+                     ? turn(g[u][t], -bd.d * kz[u][t])
+                     : make_float2(0.0f, 0.0f);
+        Dft<R, true>::run(x);
+        store_inner<R>(lds + (b * ld + q / B * R), x);
+      }
+    }
+    mid_stages<B, true>(lds, ld, tab.plan, tab.tw);
+    __syncthreads();
+    float2* dst = Z + tile_off(p * C + c, ncb, cb, H, 0, 0, kFftBatch) + col0;
+    auto out = [&](int pos, int bb, int, float2 v) {
+      const unsigned r = static_cast<unsigned>(pos - r_crop);
+      if (r < static_cast<unsigned>(H)) dst[r * kFftBatch + bb] = v;
+    };
+    last_stage_any<B>(lds, ld, tab.plan, tab.tw, out);
+  }
+}
+
+// Chirp versions: a thread's butterfly of the outermost stage owns the
+// spectrum elements j + t L/16, t < 11 (one butterfly per thread).
+template <int B>
+__global__ __launch_bounds__(768, 4) void k_chirp_col_fwd(const float2* __restrict__ X,
+                                                       float2* __restrict__ Z, int P, int C,
+                                                       int H, int r_pad, int S, int s_crop,
+                                                       float sfreq, float ap, AsmFftConsts mc,
+                                                       AnyTab tab, int accumulate) {
+  float2* lds = any_lds;
+  const int M = tab.M, ld = line_stride<B>(tab.n), ncb = M / kFftBatch;
+  int c, cb, col0, k0;
+  column_block<B>(M, &c, &cb, &col0, &k0);
+  const float2* src = nullptr;
+  const int in_shift = M / 4 - r_pad;
+  auto in = [&](int pos, int bb, int) -> float2 {
+    const unsigned r = static_cast<unsigned>(pos + in_shift);
+    return r < static_cast<unsigned>(H) ? cmulf(src[r * kFftBatch + bb], tab.chirp[pos])
+                                        : make_float2(0.0f, 0.0f);
+  };
+  const int b = threadIdx.x % B, j = threadIdx.x / B, D = tab.outer;
+  float kz[kChirpSpec];
+  float2 acc[kChirpSpec];
+#pragma unroll
+  for (int t = 0; t < kChirpSpec; ++t) {
+    const int i = j + t * D;
+    acc[t] = make_float2(0.0f, 0.0f);
+    kz[t] = j < D && i < M ? kz_or_cut(mc.k[c], i, k0 + b, M, sfreq, ap) : -1.0f;
+  }
+  for (int p = 0; p < P; ++p) {
+    __syncthreads();
+    src = X + tile_off(p * C + c, ncb, cb, H, 0, 0, kFftBatch) + col0;
+    first_stage<kChirpOuter, B, kChirpField, true>(lds, ld, tab.outer, tab.tw, in);
+    chirp_middle<B, false>(lds, ld, tab.plan, tab.tw, tab.spec);
+    const Band bd = band_of(mc, p, c);
+    auto sum = [&](int pos, int, int t, float2 v) {
+      if (passes(bd, kz[t], pos, k0 + b, M, sfreq)) acc[t] = cadd(acc[t], turn(v, bd.d * kz[t]));
+    };
+    last_stage<kChirpOuter, B, kChirpSpec, true>(lds, ld, tab.outer, tab.tw, sum);
+  }
+  __syncthreads();
+  auto spectrum = [&](int, int, int t) -> float2 { return acc[t]; };
+  first_stage<kChirpOuter, B, kChirpSpec, true>(lds, ld, tab.outer, tab.tw, spectrum);
+  chirp_middle<B, true>(lds, ld, tab.plan, tab.tw, tab.spec);
+  float2* dst = Z + tile_off(c, ncb, cb, S, 0, 0, kFftBatch) + col0;
+  const int out_shift = M / 4 - s_crop;
+  auto out = [&](int pos, int bb, int, float2 v) {
+    const unsigned r = static_cast<unsigned>(pos + out_shift);
+    if (r < static_cast<unsigned>(S)) {
+      const float2 cv = tab.chirp[pos];
+      v = cmulf(v, make_float2(cv.x, -cv.y));
+      float2* o = dst + r * kFftBatch + bb;
+      *o = accumulate ? cadd(*o, v) : v;
+    }
+  };
+  last_stage<kChirpOuter, B, kChirpField, true>(lds, ld, tab.outer, tab.tw, out);
+}
+
+template <int B>
+__global__ __launch_bounds__(768, 4) void k_chirp_col_adj(const float2* __restrict__ X,
+                                                       float2* __restrict__ Z, int P, int C,
+                                                       int S, int s_pad, int H, int r_crop,
+                                                       float sfreq, float ap, AsmFftConsts mc,
+                                                       AnyTab tab) {
+  float2* lds = any_lds;
+  const int M = tab.M, ld = line_stride<B>(tab.n), ncb = M / kFftBatch;
+  int c, cb, col0, k0;
+  column_block<B>(M, &c, &cb, &col0, &k0);
+  const float2* src = X + tile_off(c, ncb, cb, S, 0, 0, kFftBatch) + col0;
+  const int in_shift = M / 4 - s_pad;
+  auto in = [&](int pos, int bb, int) -> float2 {
+    const unsigned r = static_cast<unsigned>(pos + in_shift);
+    return r < static_cast<unsigned>(S) ? cmulf(src[r * kFftBatch + bb], tab.chirp[pos])
+                                        : make_float2(0.0f, 0.0f);
+  };
+  const int b = threadIdx.x % B, j = threadIdx.x / B, D = tab.outer;
+  first_stage<kChirpOuter, B, kChirpField, true>(lds, ld, tab.outer, tab.tw, in);
+  float kz[kChirpSpec];
+  float2 g[kChirpSpec];
+#pragma unroll
+  for (int t = 0; t < kChirpSpec; ++t) {
+    const int i = j + t * D;
+    g[t] = make_float2(0.0f, 0.0f);
+    kz[t] = j < D && i < M ? kz_or_cut(mc.k[c], i, k0 + b, M, sfreq, ap) : -1.0f;
+  }
+  chirp_middle<B, false>(lds, ld, tab.plan, tab.tw, tab.spec);
+  auto keep = [&](int, int, int t, float2 v) { g[t] = v; };
+  last_stage<kChirpOuter, B, kChirpSpec, true>(lds, ld, tab.outer, tab.tw, keep);
+  for (int p = 0; p < P; ++p) {
+    __syncthreads();
+    const Band bd = band_of(mc, p, c);
+    auto spectrum = [&](int pos, int, int t) -> float2 {
+      return passes(bd, kz[t], pos, k0 + b, M, sfreq) ? turn(g[t], -bd.d * kz[t])
+                                                      : make_float2(0.0f, 0.0f);
+    };
+    first_stage<kChirpOuter, B, kChirpSpec, true>(lds, ld, tab.outer, tab.tw, spectrum);
+    chirp_middle<B, true>(lds, ld, tab.plan, tab.tw, tab.spec);
+    float2* dst = Z + tile_off(p * C + c, ncb, cb, H, 0, 0, kFftBatch) + col0;
+    const int out_shift = M / 4 - r_crop;
+    auto out = [&](int pos, int bb, int, float2 v) {
+      const unsigned r = static_cast<unsigned>(pos + out_shift);
+      if (r < static_cast<unsigned>(H)) {
+        const float2 cv = tab.chirp[pos];
+        dst[r * kFftBatch + bb] = cmulf(v, make_float2(cv.x, -cv.y));
+      }
+    };
+    last_stage<kChirpOuter, B, kChirpField, true>(lds, ld, tab.outer, tab.tw, out);
+  }
+}
+
+// -------------------------------------------------------------- host side --
+// Radices of a smooth length in forward order: the last one is 4, 8, 12 or 16
+// (whole intermediate tiles per butterfly), the fewest stages win, then the
+// larger last radix (the stage before it then spans eight elements or more),
+// then the fewer operations (small sum of radices).
+bool factor_rest(int n, int max_stages, std::vector<int>* cur, std::vector<int>* best) {
+  if (n == 1) {
+    if (best->empty() || cur->size() < best->size()) {
+      *best = *cur;
+      return true;
+    }
+    if (cur->size() == best->size()) {
+      int a = 0, b = 0;
+      for (int v : *cur) a += v;
+      for (int v : *best) b += v;
+      if (a < b) *best = *cur;
+    }
+    return true;
+  }
+  if (static_cast<int>(cur->size()) >= max_stages) return false;
+  bool any = false;
+  for (int r : {16, 12, 10, 9, 8, 7, 6, 5, 4, 3}) {
+    if (n % r) continue;
+    if (!cur->empty() && r > cur->back()) continue;  // descending: each set once
+    cur->push_back(r);
+    any |= factor_rest(n / r, max_stages, cur, best);
+    cur->pop_back();
+  }
+  return any;
+}
+std::vector<int> smooth_radices(int M) {
+  std::vector<int> best;
+  for (int last : {16, 12, 8, 4}) {
+    if (M % last) continue;
+    std::vector<int> cur, b;
+    if (M == last || !factor_rest(M / last, kAnyMaxStages - 1, &cur, &b)) continue;
+    b.push_back(last);
+    if (best.empty() || b.size() < best.size()) best = b;
+  }
+  return best;
+}
+
+// Length and radices of the chirp transform of a padded length M: 16, two or
+// three further radices, and an odd innermost one (span 1: its accesses at
+// an odd stride meet no bank conflicts), the cheapest (length x stages) that
+// holds M + M/2 - 1 points.
+std::vector<int> chirp_radices(int M) {
+  const int need = M + M / 2 - 1;
+  std::vector<int> best;
+  int64_t cost = 0;
+  auto offer = [&](const std::vector<int>& r) {
+    int64_t n = 1;
+    for (int v : r) n *= v;
+    if (n < need || n > 3 * kAnyMaxM / 2 + 256) return;
+    const int64_t c = n * static_cast<int64_t>(r.size());
+    if (best.empty() || c < cost) {
+      best = r;
+      cost = c;
+    }
+  };
+  for (int inner : {9, 7, 5, 3}) {
+    offer({kChirpOuter, inner});
+    for (int a : {16, 12, 10, 9, 8, 7, 6, 5, 4}) {
+      offer({kChirpOuter, a, inner});
+      for (int b : {16, 12, 10, 9, 8, 7, 6, 5, 4})
+        if (b <= a) offer({kChirpOuter, a, b, inner});
+    }
+  }
+  return best;
+}
+
+// Forward stages in double, for the chirp's spectrum: leaves it in the
+// transforms' digit-reversed order.
+void host_forward(std::vector<std::complex<double>>& x, const std::vector<int>& radices) {
+  const int n = static_cast<int>(x.size());
+  std::vector<std::complex<double>> root(n);
+  for (int i = 0; i < n; ++i) root[i] = std::polar(1.0, -kTwoPiD * i / n);
+  int len = n;
+  std::vector<std::complex<double>> v(16);
+  for (int R : radices) {
+    const int D = len / R, step = n / len;
+    for (int base = 0; base < n; base += len)
+      for (int lo = 0; lo < D; ++lo) {
+        for (int m = 0; m < R; ++m) {
+          std::complex<double> s = 0.0;
+          for (int t = 0; t < R; ++t)
+            s += x[base + lo + t * D] * root[static_cast<int64_t>(t) * m % R * (n / R)];
+          v[m] = s * root[static_cast<int64_t>(lo) * m * step % n];
+        }
+        for (int m = 0; m < R; ++m) x[base + lo + m * D] = v[m];
+      }
+    len = D;
+  }
+}
+
+struct AnyTables {
+  AnyTab tab;
+  bool chirp;
+  std::vector<int> radices;
+  void* mem;
+};
+std::mutex g_any_mu;
+std::map<std::pair<int, int>, AnyTables>& any_tables() {
+  static std::map<std::pair<int, int>, AnyTables> m;
+  return m;
+}
+
+// Plan, twiddles, frequencies and chirp of a padded length, built once per
+// device (at most 150 KB per length, freed by hrf_release_caches).
+int any_tables_of(int M, AnyTables* out) {
+  int dev = 0;
+  HRF_HIP(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lock(g_any_mu);
+  const auto key = std::make_pair(dev, M);
+  auto it = any_tables().find(key);
+  if (it != any_tables().end()) {
+    *out = it->second;
+    return HRF_OK;
+  }
+  AnyTables t{};
+  t.radices = smooth_radices(M);
+  t.chirp = t.radices.empty();
+  if (t.chirp) t.radices = chirp_radices(M);
+  if (t.radices.size() < 2 || t.radices.size() > kAnyMaxStages) {
+    set_error("internal: no transform for length %d", M);
+    return HRF_ERR_INVALID;
+  }
+  AnyPlan pl{};
+  pl.n = 1;
+  for (int r : t.radices) pl.n *= r;
+  pl.stages = static_cast<int>(t.radices.size());
+  const int n = pl.n;
+  std::vector<float2> tw;
+  int len = n;
+  for (int s = 0; s < pl.stages; ++s) {
+    const int R = t.radices[s], D = len / R;
+    pl.st[s] = AnyStage{R, D, static_cast<int>(tw.size()), 1.0f / static_cast<float>(D)};
+    for (int m = 1; m < R; ++m)
+      for (int lo = 0; lo < D; ++lo) {
+        const int64_t e = static_cast<int64_t>(lo) * m * (n / len) % n;
+        const double a = -kTwoPiD * static_cast<double>(e) / n;
+        tw.push_back(make_float2(static_cast<float>(std::cos(a)), static_cast<float>(std::sin(a))));
+      }
+    len = D;
+  }
+  const int inner = t.radices.back();
+  std::vector<uint16_t> freq;
+  std::vector<float2> chirp, spec;
+  if (!t.chirp) {
+    // Position = sum of digit_s D_s; frequency = sum of digit_s times the
+    // product of the radices before it.
+    for (int j = 0; j < n / inner; ++j) {
+      int pos = j * inner, f = 0, w = 1;
+      for (int s = 0; s < pl.stages; ++s) {
+        f += pos / pl.st[s].span * w;
+        pos %= pl.st[s].span;
+        w *= pl.st[s].radix;
+      }
+      freq.push_back(static_cast<uint16_t>(f));
+    }
+  } else {
+    auto c = [&](int64_t i) {  // exp(-i pi i^2 / M), the square modulo 2M
+      const int64_t e = i * i % (2 * static_cast<int64_t>(M));
+      return std::polar(1.0, -0.5 * kTwoPiD * static_cast<double>(e) / M);
+    };
+    for (int i = 0; i < M / 2; ++i) {
+      const std::complex<double> v = c(M / 4 + i);
+      chirp.push_back(make_float2(static_cast<float>(v.real()), static_cast<float>(v.imag())));
+    }
+    // Lags l = k - n' in (-M/2, M): conj(c)(l - M/4).
+    std::vector<std::complex<double>> f(n, 0.0);
+    for (int l = -(M / 2 - 1); l < M; ++l) f[(l + n) % n] = std::conj(c(l - M / 4));
+    host_forward(f, t.radices);
+    for (const auto& v : f)
+      spec.push_back(make_float2(static_cast<float>(v.real() / n), static_cast<float>(v.imag() / n)));
+  }
+  Carver size(nullptr);
+  auto carve = [&](Carver& cv, AnyTab* tab) {
+    tab->plan = cv.take<AnyPlan>(1);
+    tab->tw = cv.take<float2>(tw.size());
+    tab->freq = cv.take<uint16_t>(freq.size() + 1);
+    tab->chirp = cv.take<float2>(chirp.size() + 1);
+    tab->spec = cv.take<float2>(spec.size() + 1);
+  };
+  carve(size, &t.tab);
+  HRF_HIP(hipMalloc(&t.mem, size.bytes()));
+  Carver cv(t.mem);
+  carve(cv, &t.tab);
+  auto put = [&](const void* dst, const void* src, size_t bytes) -> int {
+    if (bytes) HRF_HIP(hipMemcpy(const_cast<void*>(dst), src, bytes, hipMemcpyHostToDevice));
+    return HRF_OK;
+  };
+  HRF_TRY(put(t.tab.plan, &pl, sizeof(pl)));
+  HRF_TRY(put(t.tab.tw, tw.data(), tw.size() * sizeof(float2)));
+  HRF_TRY(put(t.tab.freq, freq.data(), freq.size() * sizeof(uint16_t)));
+  HRF_TRY(put(t.tab.chirp, chirp.data(), chirp.size() * sizeof(float2)));
+  HRF_TRY(put(t.tab.spec, spec.data(), spec.size() * sizeof(float2)));
+  t.tab.M = M;
+  t.tab.n = n;
+  t.tab.outer = n / t.radices[0];
+  t.tab.inner = inner;
+  any_tables()[key] = t;
+  *out = t;
+  return HRF_OK;
+}
+
+// Transforms per block: four while the batch leaves three blocks' LDS per CU
+// and there are blocks for every CU, else two.
+int batch_of(int n, int64_t lines) { return n <= 1664 && lines >= 4 * 512 ? 4 : 2; }
+
+// Threads per block: the fewest idle lanes over the stages (a stage of radix
+// R runs ceil(B n / R / T) rounds of T threads), at least `least`, at most
+// `most`.
+int threads_of(const std::vector<int>& radices, int n, int B, int least, int most = 512) {
+  int best = 0;
+  int64_t cost = 0;
+  for (int T = 64; T <= most; T += 64) {
+    if (T < least) continue;
+    int64_t c = 0;
+    for (int R : radices) {
+      const int nb = B * (n / R);
+      c += static_cast<int64_t>((nb + T - 1) / T) * T * (R + 6);
+    }
+    c += c / 16 * (512 / T);  // more threads share the latency of a round
+    if (!best || c <= cost) {
+      best = T;
+      cost = c;
+    }
+  }
+  return best;
+}
+int chirp_threads(int n, int B) { return (B * (n / kChirpOuter) + 63) / 64 * 64; }
+
+template <int B>
+size_t lds_bytes(int n) {
+  return static_cast<size_t>(B) * line_stride<B>(n) * sizeof(float2);
+}
+
+template <int B>
+int rows_in_b(const AnyTables& t, const float2* src, float2* X, int nimg, int h, int w,
+              hipStream_t s) {
+  const int M = t.tab.M;
+  const dim3 grid(nimg * ((h + B - 1) / B));
+  if (t.chirp)
+    hipLaunchKernelGGL((k_chirp_rows_in<B>), grid, dim3(chirp_threads(t.tab.n, B)),
+                       lds_bytes<B>(t.tab.n), s, src, X, h, w, M / 2 - w / 2, t.tab);
+  else
+    hipLaunchKernelGGL((k_any_rows_in<B>), grid, dim3(threads_of(t.radices, M, B, 64)),
+                       lds_bytes<B>(M), s, src, X, h, w, M / 2 - w / 2, t.tab);
+  HRF_LAUNCH_CHECK();
+  return HRF_OK;
+}
+template <int B>
+int rows_out_b(const AnyTables& t, const float2* Z, float2* dst, int nimg, int h, int w,
+               hipStream_t s) {
+  const int M = t.tab.M;
+  const float scale = static_cast<float>(1.0 / (static_cast<double>(M) * M));
+  const dim3 grid(nimg * ((h + B - 1) / B));
+  if (t.chirp)
+    hipLaunchKernelGGL((k_chirp_rows_out<B>), grid, dim3(chirp_threads(t.tab.n, B)),
+                       lds_bytes<B>(t.tab.n), s, Z, dst, h, w, M / 2 - w / 2, scale, t.tab);
+  else
+    hipLaunchKernelGGL((k_any_rows_out<B>), grid, dim3(threads_of(t.radices, M, B, 64)),
+                       lds_bytes<B>(M), s, Z, dst, h, w, M / 2 - w / 2, scale, t.tab);
+  HRF_LAUNCH_CHECK();
+  return HRF_OK;
+}
+
+template <int R, int U, int B>
+int col_any(const AnyTables& t, bool adj, const float2* X, float2* Z, int P, int C, int h_in,
+            int h_out, float sfreq, float ap, const AsmFftConsts& mc, bool accumulate,
+            hipStream_t s) {
+  const int M = t.tab.M;
+  const int least = (B * (M / R) + U - 1) / U;
+  const dim3 grid(C * (M / B)), block(threads_of(t.radices, M, B, least, R == 12 ? 704 : 512));
+  if (block.x == 0) {
+    set_error("internal: column pass of %d points does not fit a block", M);
+    return HRF_ERR_INVALID;
+  }
+  if (adj)
+    hipLaunchKernelGGL((k_any_col_adj<R, U, B>), grid, block, lds_bytes<B>(M), s, X, Z, P, C,
+                       h_in, M / 2 - h_in / 2, h_out, M / 2 - h_out / 2, sfreq, ap, mc, t.tab);
+  else
+    hipLaunchKernelGGL((k_any_col_fwd<R, U, B>), grid, block, lds_bytes<B>(M), s, X, Z, P, C,
+                       h_in, M / 2 - h_in / 2, h_out, M / 2 - h_out / 2, sfreq, ap, mc, t.tab,
+                       accumulate ? 1 : 0);
+  HRF_LAUNCH_CHECK();
+  return HRF_OK;
+}
+template <int B>
+int col_b(const AnyTables& t, bool adj, const float2* X, float2* Z, int P, int C, int h_in,
+          int h_out, float sfreq, float ap, const AsmFftConsts& mc, bool accumulate,
+          hipStream_t s) {
+  const int M = t.tab.M;
+  if (t.chirp) {
+    const dim3 grid(C * (M / B)), block(chirp_threads(t.tab.n, B));
+    if (adj)
+      hipLaunchKernelGGL((k_chirp_col_adj<B>), grid, block, lds_bytes<B>(t.tab.n), s, X, Z, P, C,
+                         h_in, M / 2 - h_in / 2, h_out, M / 2 - h_out / 2, sfreq, ap, mc, t.tab);
+    else
+      hipLaunchKernelGGL((k_chirp_col_fwd<B>), grid, block, lds_bytes<B>(t.tab.n), s, X, Z, P, C,
+                         h_in, M / 2 - h_in / 2, h_out, M / 2 - h_out / 2, sfreq, ap, mc, t.tab,
+                         accumulate ? 1 : 0);
+    HRF_LAUNCH_CHECK();
+    return HRF_OK;
+  }
+  switch (t.tab.inner) {
+    case 16:
+      return col_any<16, 1, B>(t, adj, X, Z, P, C, h_in, h_out, sfreq, ap, mc, accumulate, s);
+    case 12:
+      return col_any<12, 1, B>(t, adj, X, Z, P, C, h_in, h_out, sfreq, ap, mc, accumulate, s);
+    case 8:
+      return col_any<8, 2, B>(t, adj, X, Z, P, C, h_in, h_out, sfreq, ap, mc, accumulate, s);
+    default:
+      return col_any<4, 4, B>(t, adj, X, Z, P, C, h_in, h_out, sfreq, ap, mc, accumulate, s);
+  }
+}
+
+int rows_in(const AnyTables& t, const float2* src, float2* X, int nimg, int h, int w,
+            hipStream_t s) {
+  HRF_STAGE("asm_rows_in", s);
+  return batch_of(t.tab.n, static_cast<int64_t>(nimg) * h) == 4
+             ? rows_in_b<4>(t, src, X, nimg, h, w, s)
+             : rows_in_b<2>(t, src, X, nimg, h, w, s);
+}
+int rows_out(const AnyTables& t, const float2* Z, float2* dst, int nimg, int h, int w,
+             hipStream_t s) {
+  HRF_STAGE("asm_rows_out", s);
+  return batch_of(t.tab.n, static_cast<int64_t>(nimg) * h) == 4
+             ? rows_out_b<4>(t, Z, dst, nimg, h, w, s)
+             : rows_out_b<2>(t, Z, dst, nimg, h, w, s);
+}
+int cols(const AnyTables& t, bool adj, const float2* X, float2* Z, int P, int C, int h_in,
+         int h_out, float sfreq, float ap, const AsmFftConsts& mc, bool accumulate,
+         hipStream_t s) {
+  HRF_STAGE(adj ? "asm_col_adj" : "asm_col_fwd", s);
+  return batch_of(t.tab.n, static_cast<int64_t>(C) * t.tab.M) == 4
+             ? col_b<4>(t, adj, X, Z, P, C, h_in, h_out, sfreq, ap, mc, accumulate, s)
+             : col_b<2>(t, adj, X, Z, P, C, h_in, h_out, sfreq, ap, mc, accumulate, s);
+}
+
+}  // namespace
+
+// Both paths of this file beat the library path at every length measured
+// (table above), so the only lengths left to it are those outside the plans'
+// range and fields the chirp transforms cannot hold.
+bool any_fft_supported(int M, int H, int W) {
+  if (M < kAnyMinM || M > kAnyMaxM || M % 4 != 0) return false;
+  // The chirp transforms hold fields of at most half the grid.
+  return (2 * H <= M && 2 * W <= M) || !smooth_radices(M).empty();
+}
+
+int any_asm_forward(const float2* fields, int P, int C, int H, int W, int S, double pitch,
+                    const float* wl, const float* dist, float ap, float2* holo, float2* X,
+                    float2* Z, hipStream_t s) {
+  AnyTables t;
+  HRF_TRY(any_tables_of(2 * S, &t));
+  const AsmFftConsts mc = fft_consts(P, C, 2 * S, pitch, wl, dist);
+  HRF_TRY(rows_in(t, fields, X, P * C, H, W, s));
+  HRF_TRY(cols(t, false, X, Z, P, C, H, S, freq_step_of(2 * S, pitch), ap, mc, false, s));
+  return rows_out(t, Z, holo, C, S, S, s);
+}
+
+int any_asm_adjoint(const float2* gholo, int P, int C, int H, int W, int S, double pitch,
+                    const float* wl, const float* dist, float ap, float2* gfields, float2* X,
+                    float2* Z, hipStream_t s) {
+  AnyTables t;
+  HRF_TRY(any_tables_of(2 * S, &t));
+  const AsmFftConsts mc = fft_consts(P, C, 2 * S, pitch, wl, dist);
+  HRF_TRY(rows_in(t, gholo, X, C, S, S, s));
+  HRF_TRY(cols(t, true, X, Z, P, C, S, H, freq_step_of(2 * S, pitch), ap, mc, false, s));
+  return rows_out(t, Z, gfields, P * C, H, W, s);
+}
+
+// The multi-distance passes, grouped as in asm_fft.hip.
+int any_md_forward(const float2* field, int D, int C, int H, int W, int S, double pitch,
+                   const float* wl, const float* dist, float ap, float2* out, float2* X,
+                   float2* Z, int group, hipStream_t s) {
+  AnyTables t;
+  HRF_TRY(any_tables_of(2 * S, &t));
+  const int64_t SS = static_cast<int64_t>(S) * S;
+  HRF_TRY(rows_in(t, field, X, C, H, W, s));
+  for (int d0 = 0; d0 < D; d0 += group) {
+    const int g = D - d0 < group ? D - d0 : group;
+    const AsmFftConsts mc = fft_consts_reversed(g, C, 2 * S, pitch, wl, dist + d0);
+    HRF_TRY(cols(t, true, X, Z, g, C, H, S, freq_step_of(2 * S, pitch), ap, mc, false, s));
+    HRF_TRY(rows_out(t, Z, out + d0 * C * SS, g * C, S, S, s));
+  }
+  return HRF_OK;
+}
+
+int any_md_adjoint(const float2* gout, int D, int C, int H, int W, int S, double pitch,
+                   const float* wl, const float* dist, float ap, float2* gfield, float2* X,
+                   float2* Z, int group, hipStream_t s) {
+  AnyTables t;
+  HRF_TRY(any_tables_of(2 * S, &t));
+  const int64_t SS = static_cast<int64_t>(S) * S;
+  for (int d0 = 0; d0 < D; d0 += group) {
+    const int g = D - d0 < group ? D - d0 : group;
+    const AsmFftConsts mc = fft_consts_reversed(g, C, 2 * S, pitch, wl, dist + d0);
+    HRF_TRY(rows_in(t, gout + d0 * C * SS, X, g * C, S, S, s));
+    HRF_TRY(cols(t, false, X, Z, g, C, S, H, freq_step_of(2 * S, pitch), ap, mc, d0 > 0, s));
+  }
+  return rows_out(t, Z, gfield, C, H, W, s);
+}
+
+void any_fft_release_all() {
+  std::lock_guard<std::mutex> lock(g_any_mu);
+  for (auto& kv : any_tables()) (void)hipFree(kv.second.mem);
+  any_tables().clear();
+}
+
+}  // namespace hrf

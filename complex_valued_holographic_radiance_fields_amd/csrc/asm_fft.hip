@@ -31,14 +31,15 @@
 #include <mutex>
 #include <vector>
 
+#include "asm_common.h"
 #include "fast_trig.h"
+#include "fft_dft.h"
 #include "hrf_internal.h"
 
 namespace hrf {
 namespace {
 
 constexpr int kFftThreads = 512;   // column passes
-constexpr int kFftBatch = 4;  // columns per column-pass block; columns of an intermediate tile
 // Rows per row-pass block and its threads: four rows in 1024 threads up to
 // 1600 points, two in 512 above, where a four-row batch takes 73-147 KB of
 // LDS (two or one blocks per CU; two-row blocks measured slower at 1600).
@@ -61,273 +62,6 @@ template <int N>
 constexpr int kColBatch = N > 1600 ? 2 : kFftBatch;
 template <int N>
 constexpr int kColMinBlocks = N <= 1600 ? 4 : 2;
-constexpr double kTwoPiD = 2.0 * 3.14159265358979323846;
-
-__device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
-__device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
-// Twiddle product with explicit fused multiply-adds (the library is built
-// with contraction off for the bit-exact geometry code; the transforms only
-// need fp32 accuracy).
-__device__ __forceinline__ float2 cmulf(float2 a, float2 b) {
-  return make_float2(fmaf(a.x, b.x, -(a.y * b.y)), fmaf(a.x, b.y, a.y * b.x));
-}
-__device__ __forceinline__ float2 cscale(float2 a, float s) { return make_float2(a.x * s, a.y * s); }
-// multiply by -i (forward) or +i (inverse)
-template <bool INV>
-__device__ __forceinline__ float2 mul_mi(float2 a) {
-  return INV ? make_float2(-a.y, a.x) : make_float2(a.y, -a.x);
-}
-
-template <int R, bool INV>
-struct Dft;
-
-template <bool INV>
-struct Dft<2, INV> {
-  __device__ __forceinline__ static void run(float2 (&x)[2]) {
-    const float2 a = x[0], b = x[1];
-    x[0] = cadd(a, b);
-    x[1] = csub(a, b);
-  }
-};
-
-template <bool INV>
-struct Dft<4, INV> {
-  __device__ __forceinline__ static void run(float2 (&x)[4]) {
-    const float2 a0 = cadd(x[0], x[2]), a1 = csub(x[0], x[2]);
-    const float2 a2 = cadd(x[1], x[3]), a3 = mul_mi<INV>(csub(x[1], x[3]));
-    x[0] = cadd(a0, a2);
-    x[1] = cadd(a1, a3);
-    x[2] = csub(a0, a2);
-    x[3] = csub(a1, a3);
-  }
-};
-
-template <bool INV>
-struct Dft<8, INV> {
-  __device__ __forceinline__ static void run(float2 (&x)[8]) {
-    float2 e[4] = {x[0], x[2], x[4], x[6]};
-    float2 o[4] = {x[1], x[3], x[5], x[7]};
-    Dft<4, INV>::run(e);
-    Dft<4, INV>::run(o);
-    // o1 * e^{-/+ i pi/4} and o3 * e^{-/+ 3i pi/4}: two adds and two
-    // multiplies each.
-    constexpr float c = 0.70710678118654752f;
-    const float2 o1 = INV ? make_float2((o[1].x - o[1].y) * c, (o[1].x + o[1].y) * c)
-                          : make_float2((o[1].x + o[1].y) * c, (o[1].y - o[1].x) * c);
-    const float2 o3 = INV ? make_float2(-(o[3].x + o[3].y) * c, (o[3].x - o[3].y) * c)
-                          : make_float2((o[3].y - o[3].x) * c, -(o[3].x + o[3].y) * c);
-    const float2 o2 = mul_mi<INV>(o[2]);
-    x[0] = cadd(e[0], o[0]);
-    x[4] = csub(e[0], o[0]);
-    x[1] = cadd(e[1], o1);
-    x[5] = csub(e[1], o1);
-    x[2] = cadd(e[2], o2);
-    x[6] = csub(e[2], o2);
-    x[3] = cadd(e[3], o3);
-    x[7] = csub(e[3], o3);
-  }
-};
-
-// DFT-8 of inputs that are zero at t = 0, 1, 6, 7 (the first stage of a
-// transform whose nonzero input lies in [N/4, 3N/4)): the two DFT-4 halves
-// of (0, a, c, 0) reduce to sums and differences of a and c.
-template <bool INV>
-__device__ __forceinline__ void dft8_half(float2 (&x)[8]) {
-  const float2 a = x[2], b = x[3], c = x[4], d = x[5];
-  const float2 ma = mul_mi<INV>(a), mb = mul_mi<INV>(b);
-  float2 e[4] = {cadd(c, a), csub(ma, c), csub(c, a), csub(make_float2(-c.x, -c.y), ma)};
-  float2 o[4] = {cadd(d, b), csub(mb, d), csub(d, b), csub(make_float2(-d.x, -d.y), mb)};
-  constexpr float k = 0.70710678118654752f;
-  const float2 o1 = INV ? make_float2((o[1].x - o[1].y) * k, (o[1].x + o[1].y) * k)
-                        : make_float2((o[1].x + o[1].y) * k, (o[1].y - o[1].x) * k);
-  const float2 o3 = INV ? make_float2(-(o[3].x + o[3].y) * k, (o[3].x - o[3].y) * k)
-                        : make_float2((o[3].y - o[3].x) * k, -(o[3].x + o[3].y) * k);
-  const float2 o2 = mul_mi<INV>(o[2]);
-  x[0] = cadd(e[0], o[0]);
-  x[4] = csub(e[0], o[0]);
-  x[1] = cadd(e[1], o1);
-  x[5] = csub(e[1], o1);
-  x[2] = cadd(e[2], o2);
-  x[6] = csub(e[2], o2);
-  x[3] = cadd(e[3], o3);
-  x[7] = csub(e[3], o3);
-}
-
-// DFT-16 as two DFT-8 (even and odd inputs) combined with the twiddles
-// w16^k, k < 8.  HALF: the inputs are zero at t < 4 and t >= 12 (the
-// first stage of a transform whose nonzero input lies in [N/4, 3N/4)): the
-// even and odd halves are then both DFT-8s of inputs zero at 0, 1, 6, 7.
-template <bool INV, bool HALF>
-__device__ __forceinline__ void dft16(float2 (&x)[16]) {
-  float2 e[8], o[8];
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    if (!HALF || (j >= 2 && j <= 5)) {
-      e[j] = x[2 * j];
-      o[j] = x[2 * j + 1];
-    }
-  }
-  if constexpr (HALF) {
-    dft8_half<INV>(e);
-    dft8_half<INV>(o);
-  } else {
-    Dft<8, INV>::run(e);
-    Dft<8, INV>::run(o);
-  }
-  // o[k] * w16^k: k = 2, 6 are the DFT-8's 1/sqrt(2) products, k = 4 is
-  // -/+ i, k odd a full complex product with cos/sin(pi k/8).
-  constexpr float c1 = 0.92387953251128676f;  // cos(pi/8)
-  constexpr float s1 = 0.38268343236508977f;  // sin(pi/8)
-  constexpr float h = 0.70710678118654752f;
-  const float sg = INV ? 1.0f : -1.0f;
-  float2 t[8];
-  t[0] = o[0];
-  t[1] = cmulf(o[1], make_float2(c1, sg * s1));
-  t[2] = INV ? make_float2((o[2].x - o[2].y) * h, (o[2].x + o[2].y) * h)
-             : make_float2((o[2].x + o[2].y) * h, (o[2].y - o[2].x) * h);
-  t[3] = cmulf(o[3], make_float2(s1, sg * c1));
-  t[4] = mul_mi<INV>(o[4]);
-  t[5] = cmulf(o[5], make_float2(-s1, sg * c1));
-  t[6] = INV ? make_float2(-(o[6].x + o[6].y) * h, (o[6].x - o[6].y) * h)
-             : make_float2((o[6].y - o[6].x) * h, -(o[6].x + o[6].y) * h);
-  t[7] = cmulf(o[7], make_float2(-c1, sg * s1));
-#pragma unroll
-  for (int k = 0; k < 8; ++k) {
-    x[k] = cadd(e[k], t[k]);
-    x[k + 8] = csub(e[k], t[k]);
-  }
-}
-template <bool INV>
-struct Dft<16, INV> {
-  __device__ __forceinline__ static void run(float2 (&x)[16]) { dft16<INV, false>(x); }
-};
-
-// Odd radix by symmetric pairing: X_m = x0 + sum_j cos(2 pi jm/R)(x_j+x_{R-j})
-//   -/+ i sum_j sin(2 pi jm/R)(x_j-x_{R-j}),  X_{R-m} with the opposite sign.
-template <int R>
-struct OddConsts;
-template <>
-struct OddConsts<3> {
-  // only k = 1 occurs for R = 3 (j = m = 1)
-  __device__ static constexpr float c(int) { return -0.5f; }
-  __device__ static constexpr float s(int) { return 0.86602540378443865f; }
-};
-template <>
-struct OddConsts<5> {
-  // index (j*m) mod 5 in 1..4 -> cos/sin(2 pi k / 5)
-  __device__ static constexpr float c(int k) {
-    return (k == 1 || k == 4) ? 0.30901699437494742f : -0.80901699437494742f;
-  }
-  __device__ static constexpr float s(int k) {
-    return k == 1 ? 0.95105651629515357f
-                  : (k == 2 ? 0.58778525229247313f
-                            : (k == 3 ? -0.58778525229247313f : -0.95105651629515357f));
-  }
-};
-template <>
-struct OddConsts<7> {
-  __device__ static constexpr float c(int k) {
-    return (k == 1 || k == 6) ? 0.62348980185873353f
-                              : ((k == 2 || k == 5) ? -0.22252093395631440f : -0.90096886790241913f);
-  }
-  __device__ static constexpr float s(int k) {
-    return k == 1 ? 0.78183148246802981f
-                  : (k == 2 ? 0.97492791218182361f
-                            : (k == 3 ? 0.43388373911755812f
-                                      : (k == 4 ? -0.43388373911755812f
-                                                : (k == 5 ? -0.97492791218182361f
-                                                          : -0.78183148246802981f))));
-  }
-};
-
-template <>
-struct OddConsts<9> {
-  // cos/sin(2 pi k / 9), k = 0..8 (9 is not prime: j m = 9 at j = m = 3
-  // gives k = 0): c(9 - k) = c(k), s(9 - k) = -s(k)
-  __device__ static constexpr float c(int k) {
-    return k == 0 ? 1.0f
-           : (k == 1 || k == 8) ? 0.76604444311897804f
-                              : ((k == 2 || k == 7) ? 0.17364817766693035f
-                                                    : ((k == 3 || k == 6) ? -0.5f
-                                                                          : -0.93969262078590838f));
-  }
-  __device__ static constexpr float s(int k) {
-    return k == 0   ? 0.0f
-           : k == 1 ? 0.64278760968653933f
-           : k == 2 ? 0.98480775301220806f
-           : k == 3 ? 0.86602540378443865f
-           : k == 4 ? 0.34202014332566873f
-           : k == 5 ? -0.34202014332566873f
-           : k == 6 ? -0.86602540378443865f
-           : k == 7 ? -0.98480775301220806f
-                    : -0.64278760968653933f;
-  }
-};
-
-template <int R, bool INV>
-struct DftOdd {
-  __device__ __forceinline__ static void run(float2 (&x)[R]) {
-    constexpr int H = (R - 1) / 2;
-    float2 sp[H + 1], dm[H + 1];
-    float2 x0 = x[0];
-    float2 X0 = x0;
-#pragma unroll
-    for (int j = 1; j <= H; ++j) {
-      sp[j] = cadd(x[j], x[R - j]);
-      dm[j] = csub(x[j], x[R - j]);
-      X0 = cadd(X0, sp[j]);
-    }
-    float2 out[R];
-    out[0] = X0;
-#pragma unroll
-    for (int m = 1; m <= H; ++m) {
-      float2 re = x0, im = make_float2(0.0f, 0.0f);
-#pragma unroll
-      for (int j = 1; j <= H; ++j) {
-        const int k = (j * m) % R;
-        re = make_float2(fmaf(OddConsts<R>::c(k), sp[j].x, re.x), fmaf(OddConsts<R>::c(k), sp[j].y, re.y));
-        im = make_float2(fmaf(OddConsts<R>::s(k), dm[j].x, im.x), fmaf(OddConsts<R>::s(k), dm[j].y, im.y));
-      }
-      // X_m = re - i*im (forward), X_{R-m} = re + i*im
-      const float2 mi = mul_mi<INV>(im);
-      out[m] = cadd(re, mi);
-      out[R - m] = csub(re, mi);
-    }
-#pragma unroll
-    for (int t = 0; t < R; ++t) x[t] = out[t];
-  }
-};
-template <bool INV>
-struct Dft<3, INV> : DftOdd<3, INV> {};
-template <bool INV>
-struct Dft<5, INV> : DftOdd<5, INV> {};
-template <bool INV>
-struct Dft<7, INV> : DftOdd<7, INV> {};
-template <bool INV>
-struct Dft<9, INV> : DftOdd<9, INV> {};
-// DFT-10 by the prime-factor mapping 10 = 2 x 5 (no inner twiddles): input
-// n = (5 n1 + 2 n2) mod 10 and output k = (5 k1 + 6 k2) mod 10, i.e. a
-// DFT-2 over (x[2j], x[2j+5 mod 10]) for each j, then a DFT-5 over each of
-// the two results.
-template <bool INV>
-struct Dft<10, INV> {
-  __device__ __forceinline__ static void run(float2 (&x)[10]) {
-    float2 a[5], b[5];
-#pragma unroll
-    for (int j = 0; j < 5; ++j) {
-      const float2 u = x[2 * j], v = x[(2 * j + 5) % 10];
-      a[j] = cadd(u, v);
-      b[j] = csub(u, v);
-    }
-    Dft<5, INV>::run(a);
-    Dft<5, INV>::run(b);
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-      x[(6 * k) % 10] = a[k];
-      x[(5 + 6 * k) % 10] = b[k];
-    }
-  }
-};
 
 // LDS layout.  A batch of B transforms of length N is interleaved: element
 // i of transform b is at B*i + b, so rows and columns share one layout and
@@ -773,58 +507,6 @@ __device__ __forceinline__ const float2* stage_twiddles(float2* s_tw,
   }
 }
 
-// Transfer-function geometry of natural-order spectral element (row i,
-// column k): frequencies as torch.fft.fftfreq float32 values and the
-// aperture on the fftshifted grid (same mapping as asm_prop.hip).
-__device__ __forceinline__ void coords(int i, int kcol, int M, float sfreq, float ap,
-                                       float* fxv, float* fyv, bool* inap) {
-  const int h = M / 2;
-  int kr = i + h;
-  if (kr >= M) kr -= M;
-  int kc = kcol + h;
-  if (kc >= M) kc -= M;
-  *fxv = static_cast<float>(kr - h) * sfreq;
-  *fyv = static_cast<float>(kc - h) * sfreq;
-  bool a = true;
-  if (ap > 0.0f) {
-    const float off = static_cast<float>(M) / 2.0f - 0.5f;
-    const float x = static_cast<float>(kc) - off;
-    const float y = static_cast<float>(kr) - off;
-    a = x * x + y * y < ap * ap;
-  }
-  *inap = a;
-}
-
-// kz^2 and kz exactly as the reference kernel evaluates them
-// (bandlimited_propagation_cuda.cu:60,65-67); kz2 <= 0 -> evanescent.
-__device__ __forceinline__ float kz_of(float k, float fxv, float fyv, bool* prop) {
-  const double a = kTwoPiD * static_cast<double>(fxv);
-  const double b = kTwoPiD * static_cast<double>(fyv);
-  const float kz2 = static_cast<float>((static_cast<double>(k * k) - a * a) - b * b);
-  *prop = kz2 > 0.0f;
-  return *prop ? sqrtf(kz2) : 0.0f;
-}
-
-struct AsmFftConsts {
-  float k[kMaxChannels];
-  float d[kMaxPlanes];
-  float fxmax[kMaxPlanes * kMaxChannels];
-  float fymax[kMaxPlanes * kMaxChannels];
-  // 1 when the band limit of (plane, channel) passes every frequency of the
-  // grid (decided on the host with the device's float arithmetic), so the
-  // per-element test can be skipped.
-  unsigned char band_all[kMaxPlanes * kMaxChannels];
-};
-
-// Intermediate spectra are stored tile-major: image `img` (h rows of N
-// columns) as N/B column tiles, each h x B with the B columns innermost, at
-// ((img * N/B + tile) * h + row) * B + col.  A column pass then reads and
-// writes one contiguous h*B*8-byte run per tile, and a row pass touches
-// B*B*8 = 128-byte runs.
-__device__ __forceinline__ int64_t tile_off(int img, int ncb, int cb, int h, int r, int b, int B) {
-  return ((static_cast<int64_t>(img) * ncb + cb) * h + r) * B + b;
-}
-
 // A / A': forward FFT of kRowBatch rows of a plain (nimg, h, w_in) image
 // placed at column c_in of the zero-padded N-length row -> tiled (nimg, h,
 // N).  HALF: [c_in, c_in + w_in) lies in [N/4, 3N/4); only that half is
@@ -898,16 +580,6 @@ __global__ __launch_bounds__(kRowThreads<N>) void k_rows_out(const float2* __res
       drow[static_cast<int64_t>(r) * w_out + i] = cscale(v, scale);
   };
   Plan<N>::template run_in_out<true, T, false, RB>(lds, twp, in, out);
-}
-
-__device__ __forceinline__ void map_cblock(int bid, int nblk, int* chan, int* cb, int ncb) {
-  // XCD-aware: consecutive column tiles of a channel go to one XCD, so the
-  // tiles of neighbouring blocks stream through the same L2.
-  const int q = nblk >> 3, r = nblk & 7;
-  const int x = bid & 7, i = bid >> 3;
-  const int logical = (x < r) ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
-  *chan = logical / ncb;
-  *cb = logical - (*chan) * ncb;
 }
 
 // B: forward column pass for one channel and one column tile.  X tiled
@@ -1220,25 +892,6 @@ int twiddles(int N, const float2** out, bool col = false) {
   return HRF_OK;
 }
 
-AsmFftConsts fft_consts(int P, int C, int M, double pitch, const float* wl, const float* dist) {
-  AsmFftConsts mc{};
-  for (int c = 0; c < C; ++c) mc.k[c] = asm_consts(wl[c], 0.0f, static_cast<float>(pitch), M, M).k;
-  for (int p = 0; p < P; ++p) {
-    mc.d[p] = dist[p];
-    for (int c = 0; c < C; ++c) {
-      const AsmConsts a = asm_consts(wl[c], dist[p], static_cast<float>(pitch), M, M);
-      mc.fxmax[p * kMaxChannels + c] = a.fx_max;
-      mc.fymax[p * kMaxChannels + c] = a.fy_max;
-      // |fx| on the grid is at most float(M/2) * (float)(1/(M*pitch)), the
-      // value of the most negative bin; the device tests |f| < f_max.
-      const float fmax_grid = static_cast<float>(M / 2) *
-                              static_cast<float>(1.0 / (static_cast<double>(M) * pitch));
-      mc.band_all[p * kMaxChannels + c] = (fmax_grid < a.fx_max && fmax_grid < a.fy_max) ? 1 : 0;
-    }
-  }
-  return mc;
-}
-
 // Launches of the four passes for a length-N plan.  Inputs of width w (or
 // height h) sit centred in the padded length-N line, at N/2 - w/2; when
 // 2w <= N they lie in [N/4, 3N/4) and the pruned first stage is taken.
@@ -1304,21 +957,6 @@ int pass_col_adj(const float2* X, float2* Z, int P, int C, int h_in, int h_out, 
                        N / 2 - h_in / 2, h_out, N / 2 - h_out / 2, sfreq, ap, mc, tw);
   HRF_LAUNCH_CHECK();
   return HRF_OK;
-}
-
-float freq_step_of(int N, double pitch) {
-  return static_cast<float>(1.0 / (static_cast<double>(N) * pitch));
-}
-
-// The transfer constants with the propagation direction reversed: k_col_fwd
-// applies exp(+i d kz) and k_col_adj exp(-i d kz), so negated distances give
-// the conjugate transfer function in the one and the plain one in the other.
-// The band limits depend on d^2 and stay those of the given distances.
-AsmFftConsts fft_consts_reversed(int P, int C, int M, double pitch, const float* wl,
-                                 const float* dist) {
-  AsmFftConsts mc = fft_consts(P, C, M, pitch, wl, dist);
-  for (int p = 0; p < P; ++p) mc.d[p] = -mc.d[p];
-  return mc;
 }
 
 template <int N>

@@ -1,0 +1,361 @@
+// fft_dft.h — complex arithmetic and the R-point DFTs in registers of the LDS
+// transforms (forward e^{-i}, INV: e^{+i}, neither scaled).
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+namespace hrf {
+namespace {
+
+__device__ __forceinline__ float2 cadd(float2 a, float2 b) { return make_float2(a.x + b.x, a.y + b.y); }
+__device__ __forceinline__ float2 csub(float2 a, float2 b) { return make_float2(a.x - b.x, a.y - b.y); }
+// Twiddle product with explicit fused multiply-adds (the library is built
+// with contraction off for the bit-exact geometry code; the transforms only
+// need fp32 accuracy).
+__device__ __forceinline__ float2 cmulf(float2 a, float2 b) {
+  return make_float2(fmaf(a.x, b.x, -(a.y * b.y)), fmaf(a.x, b.y, a.y * b.x));
+}
+__device__ __forceinline__ float2 cscale(float2 a, float s) { return make_float2(a.x * s, a.y * s); }
+// multiply by -i (forward) or +i (inverse)
+template <bool INV>
+__device__ __forceinline__ float2 mul_mi(float2 a) {
+  return INV ? make_float2(-a.y, a.x) : make_float2(a.y, -a.x);
+}
+
+template <int R, bool INV>
+struct Dft;
+
+template <bool INV>
+struct Dft<2, INV> {
+  __device__ __forceinline__ static void run(float2 (&x)[2]) {
+    const float2 a = x[0], b = x[1];
+    x[0] = cadd(a, b);
+    x[1] = csub(a, b);
+  }
+};
+
+template <bool INV>
+struct Dft<4, INV> {
+  __device__ __forceinline__ static void run(float2 (&x)[4]) {
+    const float2 a0 = cadd(x[0], x[2]), a1 = csub(x[0], x[2]);
+    const float2 a2 = cadd(x[1], x[3]), a3 = mul_mi<INV>(csub(x[1], x[3]));
+    x[0] = cadd(a0, a2);
+    x[1] = cadd(a1, a3);
+    x[2] = csub(a0, a2);
+    x[3] = csub(a1, a3);
+  }
+};
+
+template <bool INV>
+struct Dft<8, INV> {
+  __device__ __forceinline__ static void run(float2 (&x)[8]) {
+    float2 e[4] = {x[0], x[2], x[4], x[6]};
+    float2 o[4] = {x[1], x[3], x[5], x[7]};
+    Dft<4, INV>::run(e);
+    Dft<4, INV>::run(o);
+    // o1 * e^{-/+ i pi/4} and o3 * e^{-/+ 3i pi/4}: two adds and two
+    // multiplies each.
+    constexpr float c = 0.70710678118654752f;
+    const float2 o1 = INV ? make_float2((o[1].x - o[1].y) * c, (o[1].x + o[1].y) * c)
+                          : make_float2((o[1].x + o[1].y) * c, (o[1].y - o[1].x) * c);
+    const float2 o3 = INV ? make_float2(-(o[3].x + o[3].y) * c, (o[3].x - o[3].y) * c)
+                          : make_float2((o[3].y - o[3].x) * c, -(o[3].x + o[3].y) * c);
+    const float2 o2 = mul_mi<INV>(o[2]);
+    x[0] = cadd(e[0], o[0]);
+    x[4] = csub(e[0], o[0]);
+    x[1] = cadd(e[1], o1);
+    x[5] = csub(e[1], o1);
+    x[2] = cadd(e[2], o2);
+    x[6] = csub(e[2], o2);
+    x[3] = cadd(e[3], o3);
+    x[7] = csub(e[3], o3);
+  }
+};
+
+// DFT-8 of inputs that are zero at t = 0, 1, 6, 7 (the first stage of a
+// transform whose nonzero input lies in [N/4, 3N/4)): the two DFT-4 halves
+// of (0, a, c, 0) reduce to sums and differences of a and c.
+template <bool INV>
+__device__ __forceinline__ void dft8_half(float2 (&x)[8]) {
+  const float2 a = x[2], b = x[3], c = x[4], d = x[5];
+  const float2 ma = mul_mi<INV>(a), mb = mul_mi<INV>(b);
+  float2 e[4] = {cadd(c, a), csub(ma, c), csub(c, a), csub(make_float2(-c.x, -c.y), ma)};
+  float2 o[4] = {cadd(d, b), csub(mb, d), csub(d, b), csub(make_float2(-d.x, -d.y), mb)};
+  constexpr float k = 0.70710678118654752f;
+  const float2 o1 = INV ? make_float2((o[1].x - o[1].y) * k, (o[1].x + o[1].y) * k)
+                        : make_float2((o[1].x + o[1].y) * k, (o[1].y - o[1].x) * k);
+  const float2 o3 = INV ? make_float2(-(o[3].x + o[3].y) * k, (o[3].x - o[3].y) * k)
+                        : make_float2((o[3].y - o[3].x) * k, -(o[3].x + o[3].y) * k);
+  const float2 o2 = mul_mi<INV>(o[2]);
+  x[0] = cadd(e[0], o[0]);
+  x[4] = csub(e[0], o[0]);
+  x[1] = cadd(e[1], o1);
+  x[5] = csub(e[1], o1);
+  x[2] = cadd(e[2], o2);
+  x[6] = csub(e[2], o2);
+  x[3] = cadd(e[3], o3);
+  x[7] = csub(e[3], o3);
+}
+
+// DFT-16 as two DFT-8 (even and odd inputs) combined with the twiddles
+// w16^k, k < 8.  HALF: the inputs are zero at t < 4 and t >= 12 (the
+// first stage of a transform whose nonzero input lies in [N/4, 3N/4)): the
+// even and odd halves are then both DFT-8s of inputs zero at 0, 1, 6, 7.
+template <bool INV, bool HALF>
+__device__ __forceinline__ void dft16(float2 (&x)[16]) {
+  float2 e[8], o[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    if (!HALF || (j >= 2 && j <= 5)) {
+      e[j] = x[2 * j];
+      o[j] = x[2 * j + 1];
+    }
+  }
+  if constexpr (HALF) {
+    dft8_half<INV>(e);
+    dft8_half<INV>(o);
+  } else {
+    Dft<8, INV>::run(e);
+    Dft<8, INV>::run(o);
+  }
+  // o[k] * w16^k: k = 2, 6 are the DFT-8's 1/sqrt(2) products, k = 4 is
+  // -/+ i, k odd a full complex product with cos/sin(pi k/8).
+  constexpr float c1 = 0.92387953251128676f;  // cos(pi/8)
+  constexpr float s1 = 0.38268343236508977f;  // sin(pi/8)
+  constexpr float h = 0.70710678118654752f;
+  const float sg = INV ? 1.0f : -1.0f;
+  float2 t[8];
+  t[0] = o[0];
+  t[1] = cmulf(o[1], make_float2(c1, sg * s1));
+  t[2] = INV ? make_float2((o[2].x - o[2].y) * h, (o[2].x + o[2].y) * h)
+             : make_float2((o[2].x + o[2].y) * h, (o[2].y - o[2].x) * h);
+  t[3] = cmulf(o[3], make_float2(s1, sg * c1));
+  t[4] = mul_mi<INV>(o[4]);
+  t[5] = cmulf(o[5], make_float2(-s1, sg * c1));
+  t[6] = INV ? make_float2(-(o[6].x + o[6].y) * h, (o[6].x - o[6].y) * h)
+             : make_float2((o[6].y - o[6].x) * h, -(o[6].x + o[6].y) * h);
+  t[7] = cmulf(o[7], make_float2(-c1, sg * s1));
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    x[k] = cadd(e[k], t[k]);
+    x[k + 8] = csub(e[k], t[k]);
+  }
+}
+template <bool INV>
+struct Dft<16, INV> {
+  __device__ __forceinline__ static void run(float2 (&x)[16]) { dft16<INV, false>(x); }
+};
+
+// Odd radix by symmetric pairing: X_m = x0 + sum_j cos(2 pi jm/R)(x_j+x_{R-j})
+//   -/+ i sum_j sin(2 pi jm/R)(x_j-x_{R-j}),  X_{R-m} with the opposite sign.
+template <int R>
+struct OddConsts;
+template <>
+struct OddConsts<3> {
+  // only k = 1 occurs for R = 3 (j = m = 1)
+  __device__ static constexpr float c(int) { return -0.5f; }
+  __device__ static constexpr float s(int) { return 0.86602540378443865f; }
+};
+template <>
+struct OddConsts<5> {
+  // index (j*m) mod 5 in 1..4 -> cos/sin(2 pi k / 5)
+  __device__ static constexpr float c(int k) {
+    return (k == 1 || k == 4) ? 0.30901699437494742f : -0.80901699437494742f;
+  }
+  __device__ static constexpr float s(int k) {
+    return k == 1 ? 0.95105651629515357f
+                  : (k == 2 ? 0.58778525229247313f
+                            : (k == 3 ? -0.58778525229247313f : -0.95105651629515357f));
+  }
+};
+template <>
+struct OddConsts<7> {
+  __device__ static constexpr float c(int k) {
+    return (k == 1 || k == 6) ? 0.62348980185873353f
+                              : ((k == 2 || k == 5) ? -0.22252093395631440f : -0.90096886790241913f);
+  }
+  __device__ static constexpr float s(int k) {
+    return k == 1 ? 0.78183148246802981f
+                  : (k == 2 ? 0.97492791218182361f
+                            : (k == 3 ? 0.43388373911755812f
+                                      : (k == 4 ? -0.43388373911755812f
+                                                : (k == 5 ? -0.97492791218182361f
+                                                          : -0.78183148246802981f))));
+  }
+};
+
+template <>
+struct OddConsts<9> {
+  // cos/sin(2 pi k / 9), k = 0..8 (9 is not prime: j m = 9 at j = m = 3
+  // gives k = 0): c(9 - k) = c(k), s(9 - k) = -s(k)
+  __device__ static constexpr float c(int k) {
+    return k == 0 ? 1.0f
+           : (k == 1 || k == 8) ? 0.76604444311897804f
+                              : ((k == 2 || k == 7) ? 0.17364817766693035f
+                                                    : ((k == 3 || k == 6) ? -0.5f
+                                                                          : -0.93969262078590838f));
+  }
+  __device__ static constexpr float s(int k) {
+    return k == 0   ? 0.0f
+           : k == 1 ? 0.64278760968653933f
+           : k == 2 ? 0.98480775301220806f
+           : k == 3 ? 0.86602540378443865f
+           : k == 4 ? 0.34202014332566873f
+           : k == 5 ? -0.34202014332566873f
+           : k == 6 ? -0.86602540378443865f
+           : k == 7 ? -0.98480775301220806f
+                    : -0.64278760968653933f;
+  }
+};
+
+template <>
+struct OddConsts<11> {
+  __device__ static constexpr float c(int k) {
+    return (k == 1 || k == 10) ? 0.84125353283118121f
+           : (k == 2 || k == 9) ? 0.41541501300188644f
+           : (k == 3 || k == 8) ? -0.142314838273285f
+           : (k == 4 || k == 7) ? -0.65486073394528499f
+           : -0.95949297361449737f;
+  }
+  __device__ static constexpr float s(int k) {
+    return k > 5 ? -s(11 - k)
+           : k == 1 ? 0.54064081745559756f
+           : k == 2 ? 0.90963199535451833f
+           : k == 3 ? 0.9898214418809328f
+           : k == 4 ? 0.75574957435425827f
+           : 0.28173255684142967f;
+  }
+};
+template <>
+struct OddConsts<13> {
+  __device__ static constexpr float c(int k) {
+    return (k == 1 || k == 12) ? 0.88545602565320991f
+           : (k == 2 || k == 11) ? 0.56806474673115592f
+           : (k == 3 || k == 10) ? 0.12053668025532301f
+           : (k == 4 || k == 9) ? -0.35460488704253545f
+           : (k == 5 || k == 8) ? -0.74851074817110119f
+           : -0.97094181742605201f;
+  }
+  __device__ static constexpr float s(int k) {
+    return k > 6 ? -s(13 - k)
+           : k == 1 ? 0.46472317204376851f
+           : k == 2 ? 0.82298386589365635f
+           : k == 3 ? 0.99270887409805397f
+           : k == 4 ? 0.93501624268541483f
+           : k == 5 ? 0.66312265824079519f
+           : 0.23931566428755768f;
+  }
+};
+
+template <int R, bool INV>
+struct DftOdd {
+  __device__ __forceinline__ static void run(float2 (&x)[R]) {
+    constexpr int H = (R - 1) / 2;
+    float2 sp[H + 1], dm[H + 1];
+    float2 x0 = x[0];
+    float2 X0 = x0;
+#pragma unroll
+    for (int j = 1; j <= H; ++j) {
+      sp[j] = cadd(x[j], x[R - j]);
+      dm[j] = csub(x[j], x[R - j]);
+      X0 = cadd(X0, sp[j]);
+    }
+    float2 out[R];
+    out[0] = X0;
+#pragma unroll
+    for (int m = 1; m <= H; ++m) {
+      float2 re = x0, im = make_float2(0.0f, 0.0f);
+#pragma unroll
+      for (int j = 1; j <= H; ++j) {
+        const int k = (j * m) % R;
+        re = make_float2(fmaf(OddConsts<R>::c(k), sp[j].x, re.x), fmaf(OddConsts<R>::c(k), sp[j].y, re.y));
+        im = make_float2(fmaf(OddConsts<R>::s(k), dm[j].x, im.x), fmaf(OddConsts<R>::s(k), dm[j].y, im.y));
+      }
+      // X_m = re - i*im (forward), X_{R-m} = re + i*im
+      const float2 mi = mul_mi<INV>(im);
+      out[m] = cadd(re, mi);
+      out[R - m] = csub(re, mi);
+    }
+#pragma unroll
+    for (int t = 0; t < R; ++t) x[t] = out[t];
+  }
+};
+template <bool INV>
+struct Dft<3, INV> : DftOdd<3, INV> {};
+template <bool INV>
+struct Dft<5, INV> : DftOdd<5, INV> {};
+template <bool INV>
+struct Dft<7, INV> : DftOdd<7, INV> {};
+template <bool INV>
+struct Dft<9, INV> : DftOdd<9, INV> {};
+template <bool INV>
+struct Dft<11, INV> : DftOdd<11, INV> {};
+template <bool INV>
+struct Dft<13, INV> : DftOdd<13, INV> {};
+// DFT-10 by the prime-factor mapping 10 = 2 x 5 (no inner twiddles): input
+// n = (5 n1 + 2 n2) mod 10 and output k = (5 k1 + 6 k2) mod 10, i.e. a
+// DFT-2 over (x[2j], x[2j+5 mod 10]) for each j, then a DFT-5 over each of
+// the two results.
+template <bool INV>
+struct Dft<10, INV> {
+  __device__ __forceinline__ static void run(float2 (&x)[10]) {
+    float2 a[5], b[5];
+#pragma unroll
+    for (int j = 0; j < 5; ++j) {
+      const float2 u = x[2 * j], v = x[(2 * j + 5) % 10];
+      a[j] = cadd(u, v);
+      b[j] = csub(u, v);
+    }
+    Dft<5, INV>::run(a);
+    Dft<5, INV>::run(b);
+#pragma unroll
+    for (int k = 0; k < 5; ++k) {
+      x[(6 * k) % 10] = a[k];
+      x[(5 + 6 * k) % 10] = b[k];
+    }
+  }
+};
+// DFT-6 and DFT-12 by the prime-factor mapping, as DFT-10: 6 = 2 x 3 with
+// input n = (3 n1 + 2 n2) mod 6 and output k = (3 k1 + 4 k2) mod 6; 12 = 4 x 3
+// with input n = (3 n1 + 4 n2) mod 12 and output k = (9 k1 + 4 k2) mod 12.
+template <bool INV>
+struct Dft<6, INV> {
+  __device__ __forceinline__ static void run(float2 (&x)[6]) {
+    float2 a[3], b[3];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+      const float2 u = x[2 * j], v = x[(2 * j + 3) % 6];
+      a[j] = cadd(u, v);
+      b[j] = csub(u, v);
+    }
+    Dft<3, INV>::run(a);
+    Dft<3, INV>::run(b);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      x[(4 * k) % 6] = a[k];
+      x[(3 + 4 * k) % 6] = b[k];
+    }
+  }
+};
+template <bool INV>
+struct Dft<12, INV> {
+  __device__ __forceinline__ static void run(float2 (&x)[12]) {
+    float2 y[3][4];
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) y[j][i] = x[(4 * j + 3 * i) % 12];
+      Dft<4, INV>::run(y[j]);
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      float2 z[3] = {y[0][i], y[1][i], y[2][i]};
+      Dft<3, INV>::run(z);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) x[(9 * i + 4 * k) % 12] = z[k];
+    }
+  }
+};
+
+}  // namespace
+}  // namespace hrf

@@ -1032,6 +1032,11 @@ int hrf_asm_multiplane_forward(const void* fields, int32_t planes, int32_t chann
                              width, size, pixel_pitch, wavelengths, distances, aperture,
                              static_cast<float2*>(hologram), spec, outs, s);
   }
+  if (any_fft_supported(M, height, width)) {
+    return any_asm_forward(static_cast<const float2*>(fields), planes, channels, height,
+                           width, size, pixel_pitch, wavelengths, distances, aperture,
+                           static_cast<float2*>(hologram), spec, outs, s);
+  }
   {
     HRF_STAGE("asm_pad", s);
     HRF_TRY(launch_asm_pad(static_cast<const float2*>(fields), PC, height, width, spec, M, s));
@@ -1080,6 +1085,11 @@ int hrf_asm_multiplane_adjoint(const void* grad_hologram, int32_t planes, int32_
     return fused_asm_adjoint(static_cast<const float2*>(grad_hologram), planes, channels,
                              height, width, size, pixel_pitch, wavelengths, distances, aperture,
                              static_cast<float2*>(grad_fields), gsp, spec, s);
+  }
+  if (any_fft_supported(M, height, width)) {
+    return any_asm_adjoint(static_cast<const float2*>(grad_hologram), planes, channels,
+                           height, width, size, pixel_pitch, wavelengths, distances, aperture,
+                           static_cast<float2*>(grad_fields), gsp, spec, s);
   }
   {
     HRF_STAGE("asm_pad", s);
@@ -1143,6 +1153,11 @@ int hrf_asm_multidistance_forward(const void* field, int32_t num_distances, int3
                             width, size, pixel_pitch, wavelengths, distances, aperture,
                             static_cast<float2*>(out), spec, buf, M / size, s);
   }
+  if (any_fft_supported(M, height, width)) {
+    return any_md_forward(static_cast<const float2*>(field), num_distances, channels, height,
+                          width, size, pixel_pitch, wavelengths, distances, aperture,
+                          static_cast<float2*>(out), spec, buf, M / size, s);
+  }
   // The C channel spectra are computed once and shared by every distance.
   {
     HRF_STAGE("asm_pad", s);
@@ -1199,6 +1214,11 @@ int hrf_asm_multidistance_adjoint(const void* grad_out, int32_t num_distances, i
                             height, width, size, pixel_pitch, wavelengths, distances, aperture,
                             static_cast<float2*>(grad_field), acc, buf, M / size, s);
   }
+  if (any_fft_supported(M, height, width)) {
+    return any_md_adjoint(static_cast<const float2*>(grad_out), num_distances, channels,
+                          height, width, size, pixel_pitch, wavelengths, distances, aperture,
+                          static_cast<float2*>(grad_field), acc, buf, M / size, s);
+  }
   // sum_d conj(T_d) FFT(pad g_d) in the spectral domain, one inverse FFT.
   for (int d = 0; d < num_distances; ++d) {
     {
@@ -1247,6 +1267,7 @@ int hrf_asm_adjoint(const void* grad_out, int32_t height, int32_t width, int32_t
 void hrf_release_caches(void) {
   hrf::fft_release_all();
   hrf::fused_fft_release_all();
+  hrf::any_fft_release_all();
 }
 
 }  // extern "C"

@@ -503,4 +503,21 @@ int fused_md_adjoint(const float2* gout, int D, int C, int H, int W, int S, doub
                      float2* Z, int group, hipStream_t s);
 void fused_fft_release_all();
 
+// The same passes for the padded lengths without a compiled plan
+// (asm_any.hip); H, W: the field's size.
+bool any_fft_supported(int M, int H, int W);
+int any_asm_forward(const float2* fields, int P, int C, int H, int W, int S, double pitch,
+                    const float* wl, const float* dist, float ap, float2* holo, float2* X,
+                    float2* Z, hipStream_t s);
+int any_asm_adjoint(const float2* gholo, int P, int C, int H, int W, int S, double pitch,
+                    const float* wl, const float* dist, float ap, float2* gfields, float2* X,
+                    float2* Z, hipStream_t s);
+int any_md_forward(const float2* field, int D, int C, int H, int W, int S, double pitch,
+                   const float* wl, const float* dist, float ap, float2* out, float2* X,
+                   float2* Z, int group, hipStream_t s);
+int any_md_adjoint(const float2* gout, int D, int C, int H, int W, int S, double pitch,
+                   const float* wl, const float* dist, float ap, float2* gfield, float2* X,
+                   float2* Z, int group, hipStream_t s);
+void any_fft_release_all();
+
 }  // namespace hrf

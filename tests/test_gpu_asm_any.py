@@ -1,0 +1,86 @@
+"""GPU parity of the propagation at padded lengths without a compiled plan:
+run-time radices (smooth lengths), the chirp transform (other lengths), and the
+hipFFT path for what neither takes."""
+import numpy as np
+import pytest
+
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+PITCH = 3.74e-6
+# Float32 transforms of up to 4096 points (chirp: 6400) in two passes per
+# direction and a phase exact to 2^-24 revolutions: about 5e-7 relative; the
+# oracle transforms in double.
+TOL = 2e-6
+
+
+def _field(rng, shape):
+    amp = rng.uniform(0, 1, size=shape)
+    ph = rng.uniform(0, 2 * np.pi, size=shape)
+    return (amp * np.exp(1j * ph)).astype(np.complex64)
+
+
+# id: which path and what is at its edge.
+CASES = [
+    ("smooth_smallest", 1, 1, 16, 12, 16),       # M = 32: two stages
+    ("smooth_last4", 2, 2, 26, 30, 30),          # M = 60 = 5 3 4
+    ("smooth_last8", 1, 3, 20, 28, 28),          # M = 56 = 7 8
+    ("smooth_last12", 2, 1, 54, 54, 54),         # M = 108 = 9 12
+    ("smooth_five_stages", 1, 1, 40, 70, 1458),  # M = 2916 = 4 3^6
+    ("smooth_four_wide", 3, 3, 700, 40, 700),    # many blocks: four transforms each
+    ("smooth_wide_tall", 2, 2, 96, 90, 50),      # fields beyond half the grid
+    ("smooth_long_lines", 1, 1, 30, 3600, 2000), # M = 4000, more than half the grid
+    ("chirp_smallest", 2, 2, 34, 22, 34),        # M = 68 = 4 17
+    ("chirp_two_wide", 1, 2, 62, 94, 94),        # M = 188 = 4 47
+    ("chirp_four_wide", 3, 3, 300, 482, 542),    # M = 1084 = 4 271, many blocks
+    ("chirp_longest", 1, 1, 64, 48, 2042),       # M = 4084 = 4 1021: L = 6144
+    ("chirp_needs_half_grid", 1, 1, 40, 60, 46), # W > S: hipFFT
+    ("below_smallest", 1, 1, 14, 10, 14),        # M = 28: hipFFT
+]
+
+
+@pytest.mark.parametrize("P,C,H,W,S", [c[1:] for c in CASES], ids=[c[0] for c in CASES])
+def test_any_length(hrf, oracle_mod, P, C, H, W, S):
+    import torch
+    from complex_valued_holographic_radiance_fields_amd import propagation
+
+    print(f"any length M={2 * S} P={P} C={C} {H}x{W}", flush=True)
+    rng = np.random.default_rng(S + H)
+    wl = [639e-9, 515e-9, 473e-9][:C]
+    # the band limit passes the whole grid at 0 and cuts it at the others
+    dist = [0.0, 3e-3, -9e-3][:P] if P > 1 else [2e-3]
+    f = _field(rng, (P, C, H, W))
+    ref = oracle_mod.multiplane_forward(f, wl, dist, PITCH, S, float(S))
+    got = propagation.multiplane(torch.from_numpy(f).cuda(), wl, PITCH, dist, (S, S), float(S))
+    assert rel_l2(got.cpu().numpy(), ref) < TOL
+    g = _field(rng, (C, S, S))
+    ref_adj = oracle_mod.multiplane_adjoint(g, H, W, wl, dist, PITCH, S, float(S))
+    got_adj = propagation.multiplane_adjoint(torch.from_numpy(g).cuda(), (H, W), wl, PITCH, dist,
+                                             (S, S), float(S))
+    assert rel_l2(got_adj.cpu().numpy(), ref_adj) < TOL
+
+
+@pytest.mark.parametrize("S,D", [(50, 3), (34, 5)], ids=["smooth", "chirp"])
+def test_any_length_multidistance(hrf, S, D):
+    """Groups of two distances (an odd last one) against single calls, and the
+    accumulated adjoint against the sum of single adjoints."""
+    import torch
+    from complex_valued_holographic_radiance_fields_amd import propagation
+
+    rng = np.random.default_rng(S)
+    C, H, W = 3, 30, 26
+    wl = [639e-9, 515e-9, 473e-9]
+    dist = [2e-3, 5e-4, -1e-3, 3e-3, -2.5e-4][:D]
+    f = torch.from_numpy(_field(rng, (C, H, W))).cuda()
+    out = propagation.multidistance(f, wl, PITCH, dist, (S, S), float(S)).cpu().numpy()
+    g = torch.from_numpy(_field(rng, (D, C, S, S))).cuda()
+    adj = propagation.multidistance_adjoint(g, (H, W), wl, PITCH, dist, (S, S), float(S))
+    for c in range(C):
+        total = 0
+        for d, dv in enumerate(dist):
+            one = propagation.propagate(f[c], wl[c], PITCH, dv, (S, S), float(S))
+            assert rel_l2(out[d, c], one.cpu().numpy()) < 1e-6
+            total = total + propagation.propagate_adjoint(g[d, c], (H, W), wl[c], PITCH, dv,
+                                                          (S, S), float(S)).cpu().numpy()
+        assert rel_l2(adj[c].cpu().numpy(), total) < 1e-6
