@@ -14,7 +14,7 @@
 // (the window is symmetric, so its adjoint is itself; zero padding makes the
 // adjoint's padding zero as well).
 //
-// Work decomposition: one 256-thread block per 32x32 output tile of one
+// Work decomposition: one block per 32x32 output tile of one
 // channel.  The window is separable (the 2-D weights are products of the
 // 1-D ones), so each block stages its input region with the halo in LDS,
 // runs the 11-tap filter along the rows into LDS and then along the columns:
@@ -22,6 +22,15 @@
 // statistics over the tile plus a 5-pixel halo (the support of the second
 // window), forms a, b, c there in LDS and filters them in the same way, so
 // it needs no workspace and reads x, y and g once per tile.
+//
+// A thread filters four neighbouring outputs at a time, so 14 LDS reads serve
+// 44 taps, and all of a block's image loads are in flight at once.  (With one
+// output per thread the kernels were bound by LDS reads, and the backward's
+// 95 KB of LDS left one 256-thread block per CU; it now takes 68 KB.)
+// 3 x 800 x 800: map 31.8 -> 24.3 us, backward 152.5 -> 47.7 us; 3 x 1080 x 1920:
+// 81.7 -> 59.4 and 466 -> 141 us.  What is left is about evenly LDS accesses,
+// VALU issue (the halos cost the backward 2.2 times its tile) and latency
+// between the barriers.
 #include <cmath>
 
 #include "hrf_internal.h"
@@ -31,110 +40,154 @@ namespace {
 
 constexpr int kSsimTile = 32;
 constexpr int kSsimR = 5;  // window radius (11 taps)
-constexpr int kSsimThreads = 256;
+// Threads per block: of 256, 448 and 576 the fastest (backward 60, 50, 59 us at
+// 3 x 800 x 800 before the loads were batched; map the same with 256 and 384).
+constexpr int kMapThreads = 256, kBwdThreads = 448;
 
 struct SsimWeights {
   float w[2 * kSsimR + 1];
 };
 
-// 11-tap filter along a row of LDS.
-__device__ __forceinline__ float tap_row(const float* row, const SsimWeights& g) {
-  float v = 0.0f;
+// Four neighbouring outputs of the 11-tap filter: out[o] = sum_k w[k] in(o + k),
+// in(0..13) each taken once.
+constexpr int kSsimOut = 4, kSsimSpan = kSsimOut + 2 * kSsimR;
+template <class In>
+__device__ __forceinline__ void taps(const SsimWeights& g, float (&out)[kSsimOut], In in) {
 #pragma unroll
-  for (int k = 0; k < 2 * kSsimR + 1; ++k) v = fmaf(g.w[k], row[k], v);
-  return v;
+  for (int o = 0; o < kSsimOut; ++o) out[o] = 0.0f;
+#pragma unroll
+  for (int i = 0; i < kSsimSpan; ++i) {
+    const float v = in(i);
+#pragma unroll
+    for (int o = 0; o < kSsimOut; ++o)
+      if (i - o >= 0 && i - o <= 2 * kSsimR) out[o] = fmaf(g.w[i - o], v, out[o]);
+  }
 }
 
-// 11-tap filter down a column of LDS (stride ld).
-__device__ __forceinline__ float tap_col(const float* col, int ld, const SsimWeights& g) {
-  float v = 0.0f;
+// Row filter of the five statistics over `rows` rows of (x, y) pairs (pitch
+// ld) into s_h[statistic][row][column] (pitch 4 groups).
+template <int T>
+__device__ __forceinline__ void row_stats(const float2* s_xy, int ld, int rows, int groups,
+                                          const SsimWeights& g, float* s_h) {
+  const int n = rows * groups * kSsimOut;  // one statistic
+  for (int i = threadIdx.x; i < rows * groups; i += T) {
+    const int r = i / groups, c = (i - r * groups) * kSsimOut;
+    const float2* p = s_xy + r * ld + c;
+    float m1[kSsimOut] = {}, m2[kSsimOut] = {}, xx[kSsimOut] = {}, yy[kSsimOut] = {},
+          xy[kSsimOut] = {};
 #pragma unroll
-  for (int k = 0; k < 2 * kSsimR + 1; ++k) v = fmaf(g.w[k], col[k * ld], v);
-  return v;
+    for (int k = 0; k < kSsimSpan; ++k) {
+      const float2 v = p[k];
+      const float px = v.x * v.x, py = v.y * v.y, pr = v.x * v.y;
+#pragma unroll
+      for (int o = 0; o < kSsimOut; ++o)
+        if (k - o >= 0 && k - o <= 2 * kSsimR) {
+          const float w = g.w[k - o];
+          m1[o] = fmaf(w, v.x, m1[o]);
+          m2[o] = fmaf(w, v.y, m2[o]);
+          xx[o] = fmaf(w, px, xx[o]);
+          yy[o] = fmaf(w, py, yy[o]);
+          xy[o] = fmaf(w, pr, xy[o]);
+        }
+    }
+    float4* o = reinterpret_cast<float4*>(s_h + r * groups * kSsimOut + c);
+    o[0] = make_float4(m1[0], m1[1], m1[2], m1[3]);
+    o[n / 4] = make_float4(m2[0], m2[1], m2[2], m2[3]);
+    o[2 * (n / 4)] = make_float4(xx[0], xx[1], xx[2], xx[3]);
+    o[3 * (n / 4)] = make_float4(yy[0], yy[1], yy[2], yy[3]);
+    o[4 * (n / 4)] = make_float4(xy[0], xy[1], xy[2], xy[3]);
+  }
 }
 
 __device__ __forceinline__ float load_px(const float* img, int H, int W, int y, int x) {
   return (y >= 0 && y < H && x >= 0 && x < W) ? img[static_cast<int64_t>(y) * W + x] : 0.0f;
 }
 
-struct SsimStats {
-  float mu1, mu2, s11, s22, s12;
-};
+// Stages the (x, y) pairs of an N x N region whose corner is (y0, x0), zero
+// outside the image, with pitch ld.  The loads are all in flight before the
+// first LDS store (one at a time they cost a memory latency per round).
+template <int N, int T>
+__device__ __forceinline__ void stage_pairs(const float* x, const float* y, int H, int W, int y0,
+                                            int x0, int ld, float2* s_xy) {
+  constexpr int kRounds = (N * N + T - 1) / T;
+  float2 v[kRounds];
+#pragma unroll
+  for (int u = 0; u < kRounds; ++u) {
+    const int i = threadIdx.x + u * T;
+    const int r = i / N, c = i - r * N;
+    const bool in = i < N * N;
+    v[u] = make_float2(in ? load_px(x, H, W, y0 + r, x0 + c) : 0.0f,
+                       in ? load_px(y, H, W, y0 + r, x0 + c) : 0.0f);
+  }
+#pragma unroll
+  for (int u = 0; u < kRounds; ++u) {
+    const int i = threadIdx.x + u * T;
+    const int r = i / N, c = i - r * N;
+    if (i < N * N) s_xy[r * ld + c] = v[u];
+  }
+}
 
-// The SSIM factors in the reference's evaluation order
-// (conv.cu:993-1001).
+// The SSIM factors: map = C D / (A B).
 struct SsimTerms {
   float A, B, C, D;
 };
 
-__device__ __forceinline__ SsimTerms ssim_terms(const SsimStats& st, float C1, float C2) {
+__device__ __forceinline__ SsimTerms ssim_terms(float mu1, float mu2, float xx, float yy,
+                                                float xy, float C1, float C2) {
   SsimTerms t;
-  const float mu1_sq = st.mu1 * st.mu1;
-  const float mu2_sq = st.mu2 * st.mu2;
-  const float mu1_mu2 = st.mu1 * st.mu2;
+  const float mu1_sq = mu1 * mu1;
+  const float mu2_sq = mu2 * mu2;
+  const float mu1_mu2 = mu1 * mu2;
   t.C = 2.0f * mu1_mu2 + C1;
-  t.D = 2.0f * st.s12 + C2;
+  t.D = 2.0f * (xy - mu1_mu2) + C2;
   t.A = mu1_sq + mu2_sq + C1;
-  t.B = st.s11 + st.s22 + C2;
+  t.B = (xx - mu1_sq) + (yy - mu2_sq) + C2;
   return t;
+}
+
+// Column filter of statistic block `s_h` (pitch ld) at rows r .. r + 3 of
+// column c.
+__device__ __forceinline__ void col_taps(const float* s_h, int ld, int r, int c,
+                                         const SsimWeights& g, float (&out)[kSsimOut]) {
+  const float* p = s_h + r * ld + c;
+  taps(g, out, [&](int i) { return p[i * ld]; });
 }
 
 // Forward: region of (32 + 10)^2 inputs -> 32 x 32 outputs.
 constexpr int kFwdIn = kSsimTile + 2 * kSsimR;  // 42
-constexpr int kFwdLd = kFwdIn + 1;              // LDS row pitch (odd: no bank aliasing)
+constexpr int kFwdLd = kFwdIn + 1;  // row pitch in pairs (odd: four rows' reads interleave)
 
-__global__ __launch_bounds__(kSsimThreads) void k_ssim_map(const float* __restrict__ img1,
+__global__ __launch_bounds__(kMapThreads) void k_ssim_map(const float* __restrict__ img1,
                                                           const float* __restrict__ img2, int H,
                                                           int W, float C1, float C2,
                                                           SsimWeights g,
                                                           float* __restrict__ map) {
-  __shared__ float s_x[kFwdIn * kFwdLd];
-  __shared__ float s_y[kFwdIn * kFwdLd];
+  __shared__ float2 s_xy[kFwdIn * kFwdLd];
   // Row-filtered statistics: 5 x (42 rows x 32 columns).
-  __shared__ float s_h[5][kFwdIn * kSsimTile];
+  constexpr int kHN = kFwdIn * kSsimTile;
+  __shared__ __align__(16) float s_h[5 * kHN];
   const int64_t plane = static_cast<int64_t>(blockIdx.z) * H * W;
   const float* x = img1 + plane;
   const float* y = img2 + plane;
   const int oy = blockIdx.y * kSsimTile, ox = blockIdx.x * kSsimTile;
-  for (int i = threadIdx.x; i < kFwdIn * kFwdIn; i += kSsimThreads) {
-    const int r = i / kFwdIn, c = i - r * kFwdIn;
-    s_x[r * kFwdLd + c] = load_px(x, H, W, oy - kSsimR + r, ox - kSsimR + c);
-    s_y[r * kFwdLd + c] = load_px(y, H, W, oy - kSsimR + r, ox - kSsimR + c);
-  }
+  stage_pairs<kFwdIn, kMapThreads>(x, y, H, W, oy - kSsimR, ox - kSsimR, kFwdLd, s_xy);
   __syncthreads();
-  for (int i = threadIdx.x; i < kFwdIn * kSsimTile; i += kSsimThreads) {
-    const int r = i / kSsimTile, c = i - r * kSsimTile;
-    const float* px = s_x + r * kFwdLd + c;
-    const float* py = s_y + r * kFwdLd + c;
-    float m1 = 0.0f, m2 = 0.0f, e11 = 0.0f, e22 = 0.0f, e12 = 0.0f;
+  row_stats<kMapThreads>(s_xy, kFwdLd, kFwdIn, kSsimTile / kSsimOut, g, s_h);
+  __syncthreads();
+  static_assert(kSsimTile * kSsimTile <= kSsimOut * kMapThreads, "one column run per thread");
+  if (threadIdx.x >= kSsimTile * kSsimTile / kSsimOut) return;
+  const int c = threadIdx.x % kSsimTile, r = threadIdx.x / kSsimTile * kSsimOut;
+  float m1[kSsimOut], m2[kSsimOut], xx[kSsimOut], yy[kSsimOut], xy[kSsimOut];
+  col_taps(s_h, kSsimTile, r, c, g, m1);
+  col_taps(s_h + kHN, kSsimTile, r, c, g, m2);
+  col_taps(s_h + 2 * kHN, kSsimTile, r, c, g, xx);
+  col_taps(s_h + 3 * kHN, kSsimTile, r, c, g, yy);
+  col_taps(s_h + 4 * kHN, kSsimTile, r, c, g, xy);
 #pragma unroll
-    for (int k = 0; k < 2 * kSsimR + 1; ++k) {
-      const float a = px[k], b = py[k], w = g.w[k];
-      m1 = fmaf(w, a, m1);
-      m2 = fmaf(w, b, m2);
-      e11 = fmaf(w, a * a, e11);
-      e22 = fmaf(w, b * b, e22);
-      e12 = fmaf(w, a * b, e12);
-    }
-    s_h[0][i] = m1;
-    s_h[1][i] = m2;
-    s_h[2][i] = e11;
-    s_h[3][i] = e22;
-    s_h[4][i] = e12;
-  }
-  __syncthreads();
-  for (int i = threadIdx.x; i < kSsimTile * kSsimTile; i += kSsimThreads) {
-    const int r = i / kSsimTile, c = i - r * kSsimTile;
-    const int py = oy + r, px = ox + c;
+  for (int o = 0; o < kSsimOut; ++o) {
+    const int py = oy + r + o, px = ox + c;
     if (py >= H || px >= W) continue;
-    const int o = r * kSsimTile + c;
-    SsimStats st;
-    st.mu1 = tap_col(s_h[0] + o, kSsimTile, g);
-    st.mu2 = tap_col(s_h[1] + o, kSsimTile, g);
-    st.s11 = tap_col(s_h[2] + o, kSsimTile, g) - st.mu1 * st.mu1;
-    st.s22 = tap_col(s_h[3] + o, kSsimTile, g) - st.mu2 * st.mu2;
-    st.s12 = tap_col(s_h[4] + o, kSsimTile, g) - st.mu1 * st.mu2;
-    const SsimTerms t = ssim_terms(st, C1, C2);
+    const SsimTerms t = ssim_terms(m1[o], m2[o], xx[o], yy[o], xy[o], C1, C2);
     map[plane + static_cast<int64_t>(py) * W + px] = (t.C * t.D) / (t.A * t.B);
   }
 }
@@ -145,99 +198,93 @@ constexpr int kBwdIn = kSsimTile + 4 * kSsimR;  // 52
 constexpr int kBwdLd = kBwdIn + 1;
 constexpr int kBwdMid = kSsimTile + 2 * kSsimR;  // 42
 constexpr int kBwdMidLd = kBwdMid + 1;
+constexpr int kBwdGroups = (kBwdMid + kSsimOut - 1) / kSsimOut;  // 11: columns 42, 43 unused
+constexpr int kBwdHLd = kBwdGroups * kSsimOut;
 
-__global__ __launch_bounds__(kSsimThreads) void k_ssim_backward(
+__global__ __launch_bounds__(kBwdThreads) void k_ssim_backward(
     const float* __restrict__ img1, const float* __restrict__ img2,
     const float* __restrict__ grad_map, int H, int W, float C1, float C2, SsimWeights g,
     float* __restrict__ grad_img1) {
-  __shared__ float s_x[kBwdIn * kBwdLd];
-  __shared__ float s_y[kBwdIn * kBwdLd];
-  // Row-filtered statistics (5 x 52 rows x 42 columns); afterwards reused
-  // for the row-filtered a, b, c (3 x 42 rows x 32 columns).
-  __shared__ float s_h[5 * kBwdIn * kBwdMid];
-  __shared__ float s_abc[3][kBwdMid * kBwdMidLd];
+  // The staged pairs (and the unused last group's reads past the last row),
+  // afterwards a, b, c over the 42 x 42 positions.
+  constexpr int kPairs = kBwdIn * kBwdLd + kSsimOut;
+  __shared__ float2 s_xy[kPairs];
+  static_assert(2 * kPairs >= 3 * kBwdMid * kBwdMidLd, "a, b, c in the pairs' place");
+  float* s_abc = reinterpret_cast<float*>(s_xy);
+  constexpr int kABC = kBwdMid * kBwdMidLd;
+  // Row-filtered statistics (5 x 52 rows x 44 columns; the unused last
+  // group's column filter reads past the last row of one block into the
+  // next), afterwards the row-filtered a, b, c (3 x 42 rows x 32 columns).
+  constexpr int kHN = kBwdIn * kBwdHLd;
+  __shared__ __align__(16) float s_h[5 * kHN + 2 * kBwdHLd];
   const int64_t plane = static_cast<int64_t>(blockIdx.z) * H * W;
   const float* x = img1 + plane;
   const float* y = img2 + plane;
   const float* gm = grad_map + plane;
   const int oy = blockIdx.y * kSsimTile, ox = blockIdx.x * kSsimTile;
-  const int y0 = oy - 2 * kSsimR, x0 = ox - 2 * kSsimR;  // input region origin
-  for (int i = threadIdx.x; i < kBwdIn * kBwdIn; i += kSsimThreads) {
-    const int r = i / kBwdIn, c = i - r * kBwdIn;
-    s_x[r * kBwdLd + c] = load_px(x, H, W, y0 + r, x0 + c);
-    s_y[r * kBwdLd + c] = load_px(y, H, W, y0 + r, x0 + c);
-  }
+  stage_pairs<kBwdIn, kBwdThreads>(x, y, H, W, oy - 2 * kSsimR, ox - 2 * kSsimR, kBwdLd, s_xy);
   __syncthreads();
-  constexpr int kHN = kBwdIn * kBwdMid;  // one statistic's row-filtered block
-  for (int i = threadIdx.x; i < kHN; i += kSsimThreads) {
-    const int r = i / kBwdMid, c = i - r * kBwdMid;
-    const float* px = s_x + r * kBwdLd + c;
-    const float* py = s_y + r * kBwdLd + c;
-    float m1 = 0.0f, m2 = 0.0f, e11 = 0.0f, e22 = 0.0f, e12 = 0.0f;
-#pragma unroll
-    for (int k = 0; k < 2 * kSsimR + 1; ++k) {
-      const float a = px[k], b = py[k], w = g.w[k];
-      m1 = fmaf(w, a, m1);
-      m2 = fmaf(w, b, m2);
-      e11 = fmaf(w, a * a, e11);
-      e22 = fmaf(w, b * b, e22);
-      e12 = fmaf(w, a * b, e12);
-    }
-    s_h[0 * kHN + i] = m1;
-    s_h[1 * kHN + i] = m2;
-    s_h[2 * kHN + i] = e11;
-    s_h[3 * kHN + i] = e22;
-    s_h[4 * kHN + i] = e12;
-  }
+  row_stats<kBwdThreads>(s_xy, kBwdLd, kBwdIn, kBwdGroups, g, s_h);
   __syncthreads();
   // Statistics at the 42 x 42 positions around the tile; a, b, c there
   // (zero outside the image, where the map has no gradient).
-  for (int i = threadIdx.x; i < kBwdMid * kBwdMid; i += kSsimThreads) {
-    const int r = i / kBwdMid, c = i - r * kBwdMid;
-    const int py = oy - kSsimR + r, px = ox - kSsimR + c;
-    float a = 0.0f, b = 0.0f, cc = 0.0f;
-    if (py >= 0 && py < H && px >= 0 && px < W) {
-      const int o = r * kBwdMid + c;
-      SsimStats st;
-      st.mu1 = tap_col(s_h + 0 * kHN + o, kBwdMid, g);
-      st.mu2 = tap_col(s_h + 1 * kHN + o, kBwdMid, g);
-      st.s11 = tap_col(s_h + 2 * kHN + o, kBwdMid, g) - st.mu1 * st.mu1;
-      st.s22 = tap_col(s_h + 3 * kHN + o, kBwdMid, g) - st.mu2 * st.mu2;
-      st.s12 = tap_col(s_h + 4 * kHN + o, kBwdMid, g) - st.mu1 * st.mu2;
-      const SsimTerms t = ssim_terms(st, C1, C2);
-      const float dm = gm[static_cast<int64_t>(py) * W + px];
-      const float AB = t.A * t.B;
-      // d map / d mu1 (the w*x^2 and w*xy statistics held fixed),
-      // d map / d(w*x^2), d map / d(w*xy)  (conv.cu:1081-1088)
-      a = dm * ((st.mu2 * 2.0f * t.D) / AB - (st.mu2 * 2.0f * t.C) / AB -
-                (st.mu1 * 2.0f * t.C * t.D) / (t.A * t.A * t.B) +
-                (st.mu1 * 2.0f * t.C * t.D) / (AB * t.B));
-      b = dm * ((-t.C * t.D) / (AB * t.B));
-      cc = dm * ((2.0f * t.C) / AB);
+  for (int i = threadIdx.x; i < kBwdGroups * kBwdMid; i += kBwdThreads) {
+    const int c = i % kBwdMid, r = i / kBwdMid * kSsimOut;
+    float m1[kSsimOut], m2[kSsimOut], xx[kSsimOut], yy[kSsimOut], xy[kSsimOut];
+    col_taps(s_h, kBwdHLd, r, c, g, m1);
+    col_taps(s_h + kHN, kBwdHLd, r, c, g, m2);
+    col_taps(s_h + 2 * kHN, kBwdHLd, r, c, g, xx);
+    col_taps(s_h + 3 * kHN, kBwdHLd, r, c, g, yy);
+    col_taps(s_h + 4 * kHN, kBwdHLd, r, c, g, xy);
+#pragma unroll
+    for (int o = 0; o < kSsimOut; ++o) {
+      if (r + o >= kBwdMid) break;
+      const int py = oy - kSsimR + r + o, px = ox - kSsimR + c;
+      float a = 0.0f, b = 0.0f, cc = 0.0f;
+      if (py >= 0 && py < H && px >= 0 && px < W) {
+        const SsimTerms t = ssim_terms(m1[o], m2[o], xx[o], yy[o], xy[o], C1, C2);
+        const float dm = gm[static_cast<int64_t>(py) * W + px];
+        const float iA = 1.0f / t.A, iB = 1.0f / t.B;
+        const float cab = dm * t.C * iA * iB;  // dm C / (A B)
+        const float map = cab * t.D;           // dm C D / (A B)
+        // d map / d mu1 (the w*x^2 and w*xy statistics held fixed),
+        // d map / d(w*x^2), d map / d(w*xy)  (conv.cu:1081-1088)
+        a = 2.0f * (m2[o] * (dm * iA * iB * t.D - cab) - m1[o] * map * (iA - iB));
+        b = -map * iB;
+        cc = 2.0f * cab;
+      }
+      s_abc[(r + o) * kBwdMidLd + c] = a;
+      s_abc[kABC + (r + o) * kBwdMidLd + c] = b;
+      s_abc[2 * kABC + (r + o) * kBwdMidLd + c] = cc;
     }
-    s_abc[0][r * kBwdMidLd + c] = a;
-    s_abc[1][r * kBwdMidLd + c] = b;
-    s_abc[2][r * kBwdMidLd + c] = cc;
   }
   __syncthreads();
   constexpr int kH2 = kBwdMid * kSsimTile;
-  for (int i = threadIdx.x; i < kH2; i += kSsimThreads) {
-    const int r = i / kSsimTile, c = i - r * kSsimTile;
+  constexpr int kGroups = kSsimTile / kSsimOut;
+  for (int i = threadIdx.x; i < kBwdMid * kGroups; i += kBwdThreads) {
+    const int r = i / kGroups, c = (i - r * kGroups) * kSsimOut;
 #pragma unroll
-    for (int q = 0; q < 3; ++q) s_h[q * kH2 + i] = tap_row(&s_abc[q][r * kBwdMidLd + c], g);
+    for (int k = 0; k < 3; ++k) {
+      const float* p = s_abc + k * kABC + r * kBwdMidLd + c;
+      float v[kSsimOut];
+      taps(g, v, [&](int j) { return p[j]; });
+      *reinterpret_cast<float4*>(s_h + k * kH2 + r * kSsimTile + c) =
+          make_float4(v[0], v[1], v[2], v[3]);
+    }
   }
   __syncthreads();
-  for (int i = threadIdx.x; i < kSsimTile * kSsimTile; i += kSsimThreads) {
-    const int r = i / kSsimTile, c = i - r * kSsimTile;
-    const int py = oy + r, px = ox + c;
+  if (threadIdx.x >= kSsimTile * kSsimTile / kSsimOut) return;
+  const int c = threadIdx.x % kSsimTile, r = threadIdx.x / kSsimTile * kSsimOut;
+  float wa[kSsimOut], wb[kSsimOut], wc[kSsimOut];
+  col_taps(s_h, kSsimTile, r, c, g, wa);
+  col_taps(s_h + kH2, kSsimTile, r, c, g, wb);
+  col_taps(s_h + 2 * kH2, kSsimTile, r, c, g, wc);
+#pragma unroll
+  for (int o = 0; o < kSsimOut; ++o) {
+    const int py = oy + r + o, px = ox + c;
     if (py >= H || px >= W) continue;
-    const int o = r * kSsimTile + c;
-    const float wa = tap_col(s_h + 0 * kH2 + o, kSsimTile, g);
-    const float wb = tap_col(s_h + 1 * kH2 + o, kSsimTile, g);
-    const float wc = tap_col(s_h + 2 * kH2 + o, kSsimTile, g);
-    const float xv = s_x[(r + 2 * kSsimR) * kBwdLd + c + 2 * kSsimR];
-    const float yv = s_y[(r + 2 * kSsimR) * kBwdLd + c + 2 * kSsimR];
-    grad_img1[plane + static_cast<int64_t>(py) * W + px] = wa + xv * (2.0f * wb) + yv * wc;
+    const int64_t at = static_cast<int64_t>(py) * W + px;
+    grad_img1[plane + at] = wa[o] + x[at] * (2.0f * wb[o]) + y[at] * wc[o];
   }
 }
 
@@ -284,7 +331,7 @@ int hrf_ssim_map(const float* img1, const float* img2, int32_t channels, int32_t
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   HRF_STAGE("ssim", s);
-  hipLaunchKernelGGL(k_ssim_map, ssim_grid(channels, height, width), dim3(kSsimThreads), 0, s,
+  hipLaunchKernelGGL(k_ssim_map, ssim_grid(channels, height, width), dim3(kMapThreads), 0, s,
                      img1, img2, height, width, c1, c2, ssim_weights(), ssim_map);
   HRF_LAUNCH_CHECK();
   return HRF_OK;
@@ -300,7 +347,7 @@ int hrf_ssim_backward(const float* img1, const float* img2, const float* grad_ma
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   HRF_STAGE("ssim", s);
-  hipLaunchKernelGGL(k_ssim_backward, ssim_grid(channels, height, width), dim3(kSsimThreads), 0,
+  hipLaunchKernelGGL(k_ssim_backward, ssim_grid(channels, height, width), dim3(kBwdThreads), 0,
                      s, img1, img2, grad_map, height, width, c1, c2, ssim_weights(), grad_img1);
   HRF_LAUNCH_CHECK();
   return HRF_OK;
