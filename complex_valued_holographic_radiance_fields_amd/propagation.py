@@ -146,6 +146,24 @@ def _floats(vals):
     return [_as_float(v) for v in (vals.tolist() if isinstance(vals, torch.Tensor) else vals)]
 
 
+# Most workspace the multi-distance calls ask for beyond what they need: room
+# for more distances per column pass.
+_MD_EXTRA_BYTES = 2 << 30
+
+
+def _md_workspace(D: int, C: int, S: int, dev) -> tuple[torch.Tensor, int]:
+    need = _lib.load().hrf_asm_multidistance_workspace_size(C, S)  # two distances a pass
+    one = 8 * C * S * 2 * S
+    more = min(min(D, 32) - 2, _MD_EXTRA_BYTES // one)
+    stream = _lib.stream_ptr(dev)
+    if more > 0:
+        try:
+            return _lib.workspace("asm_md", dev, stream, need + more * one), need + more * one
+        except torch.OutOfMemoryError:
+            pass
+    return _lib.workspace("asm_md", dev, stream, need), need
+
+
 def multidistance(fields: torch.Tensor, wavelengths, pixel_pitch, distances, size,
                   aperture_size=-1.0) -> torch.Tensor:
     """fields (C,H,W) -> (D,C,S,S) with out[d,c] = propagate(fields[c],
@@ -163,8 +181,7 @@ def multidistance(fields: torch.Tensor, wavelengths, pixel_pitch, distances, siz
     out = torch.empty((len(ds), C, S, S), dtype=torch.complex64, device=fields.device)
     lib = _lib.load()
     with torch.cuda.device(fields.device):
-        nb = lib.hrf_asm_multidistance_workspace_size(C, S)
-        ws = _lib.workspace("asm_md", fields.device, _lib.stream_ptr(fields.device), nb)
+        ws, nb = _md_workspace(len(ds), C, S, fields.device)
         _lib.check(lib.hrf_asm_multidistance_forward(
             fields.data_ptr(), len(ds), C, H, W, S, _host_f32(wl), _host_f32(ds),
             _as_float(pixel_pitch), _as_float(aperture_size), out.data_ptr(), ws.data_ptr(), nb,
@@ -187,8 +204,7 @@ def multidistance_adjoint(grad_out: torch.Tensor, field_hw, wavelengths, pixel_p
     out = torch.empty((C, H, W), dtype=torch.complex64, device=grad_out.device)
     lib = _lib.load()
     with torch.cuda.device(grad_out.device):
-        nb = lib.hrf_asm_multidistance_workspace_size(C, S)
-        ws = _lib.workspace("asm_md", grad_out.device, _lib.stream_ptr(grad_out.device), nb)
+        ws, nb = _md_workspace(D, C, S, grad_out.device)
         _lib.check(lib.hrf_asm_multidistance_adjoint(
             grad_out.data_ptr(), D, C, H, W, S, _host_f32(wl), _host_f32(ds),
             _as_float(pixel_pitch), _as_float(aperture_size), out.data_ptr(), ws.data_ptr(), nb,

@@ -298,8 +298,10 @@ int hrf_asm_multiplane_adjoint(const void* grad_hologram, int32_t planes,
  * distances[d]).  Each channel is transformed once and shared by all D
  * distances (C + D*C transforms instead of 2*D*C).  Replaces the
  * per-(distance, wavelength) BandlimitedPropagation calls of the
- * propagation microbench (python_function.py:220-226).  Any even size
- * (hipFFT transforms). */
+ * propagation microbench (python_function.py:220-226).  Any even size.
+ * The workspace size is the least; C * S * 2S * 8 bytes more for each
+ * distance beyond two let the passes take that many distances at a time
+ * (at most 32). */
 size_t hrf_asm_multidistance_workspace_size(int32_t channels, int32_t size);
 int hrf_asm_multidistance_forward(const void* fields, int32_t num_distances,
                                   int32_t channels, int32_t height, int32_t width,

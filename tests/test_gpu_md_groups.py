@@ -1,0 +1,37 @@
+"""Multi-distance propagation with as many distances per column pass as the
+workspace holds, against the least workspace (two per pass)."""
+import numpy as np
+import pytest
+
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("D", [1, 2, 3, 8, 34])
+@pytest.mark.parametrize("S", [64, 50, 34], ids=["planned", "smooth", "chirp"])
+def test_distances_per_pass(hrf, monkeypatch, S, D):
+    import torch
+    from complex_valued_holographic_radiance_fields_amd import _lib, propagation
+
+    rng = np.random.default_rng(S + D)
+    C, H, W = 2, 30, 26
+    wl = [639e-9, 473e-9]
+    dist = [float(v) for v in np.linspace(-4e-3, 5e-3, D)]
+    z = lambda *s: torch.from_numpy((rng.normal(size=s) + 1j * rng.normal(size=s))  # noqa: E731
+                                    .astype(np.complex64)).cuda()
+    f, g = z(C, H, W), z(D, C, S, S)
+    args = (wl, 3.74e-6, dist, (S, S), float(S))
+
+    def both():
+        _lib.release_workspaces()
+        return (propagation.multidistance(f, *args).cpu().numpy(),
+                propagation.multidistance_adjoint(g, (H, W), *args).cpu().numpy())
+
+    out, adj = both()
+    monkeypatch.setattr(propagation, "_MD_EXTRA_BYTES", 0)
+    out2, adj2 = both()
+    _lib.release_workspaces()
+    assert np.array_equal(out, out2)  # the same arithmetic per distance
+    # the adjoint's sum over passes is taken after the inverse transform
+    assert rel_l2(adj, adj2) < 1e-6
