@@ -222,7 +222,6 @@ struct GeomBwdParams {
 int launch_geom_backward(const GeomBwdParams& p, hipStream_t s);
 
 // Scan scratch sizing (block-sum pyramid of an n-element scan).
-size_t scan_scratch_elems(int64_t n);
 
 // Stable LSD radix sort of (u32 key, u32 value) pairs over bits
 // [0, end_bit).  Ping-pongs between (ka,va) and (kb,vb); returns in
@@ -345,15 +344,6 @@ int launch_tile_ranges_from_rects(const uint32_t* tiles, const uint2* rect, int6
                                   int gy, int32_t* diff, int32_t* ranges, hipStream_t s,
                                   int32_t* tile_order = nullptr);
 
-// Exclusive pair offsets off[0..n] (off[n] = K) of the tile counts taken in
-// depth-rank order (tiles[order[i]]; order == nullptr: index order) and
-// exclusive visible offsets vis_off (index order); totals receives
-// [K, V, *sort_flag] and, when tag != 0, totals[3] = tag after a
-// system-scope fence (the host polls it).  bsum_p / bsum_v: ceil(n / 2048) elements each.
-int launch_offsets(const uint32_t* order, const uint32_t* tiles, const uint32_t* vis,
-                   int64_t n, uint64_t* off, uint32_t* vis_off, uint64_t* bsum_p,
-                   uint32_t* bsum_v, const uint32_t* sort_flag, uint64_t* totals,
-                   hipStream_t s, uint64_t tag = 0);
 // Count partials: part_t / part_v hold per-kProjThreads-block sums (from
 // k_project, index order, part_v with the kPartFlag bits); launch_partials_scan
 // turns them, in place, into exclusive block bases (part_t[nb] = K), writes

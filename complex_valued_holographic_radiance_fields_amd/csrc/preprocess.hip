@@ -9,13 +9,24 @@
 // (model.py:41-56), and the transform in Scene.splat (model.py:1161-1162).
 // The reference runs ~15 torch ops and a global torch.sort; here the
 // selection is one kernel over the parameters in index order (transform,
-// filter and every activation, packed into one record per kept row), the
-// flag scan shared with the binning, one compaction, a stable 32-bit radix
-// sort of the selected depth keys, and one gather of the records in depth
-// order.  The backward packs the output gradients in depth order, then
-// writes every parameter-gradient row in index order, so both passes over
-// the parameter arrays are coalesced.
+// filter and every activation, packed into one record per kept row), a
+// stable radix sort of all rows' depth keys in which the dropped rows come
+// last (so nothing is compacted and the sort is queued without waiting for
+// the count), and one gather of the records in depth order.  The backward
+// packs the output gradients, read in depth order, at their parameter rows,
+// then writes every parameter-gradient row in index order, so both passes
+// over the parameter arrays are coalesced.
+//
+// Keys: a kept depth lies in (near, far), so its float bits less those of
+// max(near, 0) need only as many bits as far's do (27 for 1 .. 1000: four
+// passes of 7, 7, 7 and 6 bits instead of four of 8), and that of far itself
+// serves as every dropped row's key.
+//
+// All kernels here are bound by memory: 1M Gaussians, three planes: forward
+// 189 -> 148 us, backward 133 -> 110 us against compaction, 32-bit keys, an
+// inverse permutation in the backward and records moved by their own lanes.
 #include <cmath>
+#include <cstring>
 
 #include "hrf_internal.h"
 
@@ -53,49 +64,75 @@ __device__ __forceinline__ void to_camera(const View& v, float m0, float m1, flo
 // record with everything the depth-ordered gather needs, so the gather reads
 // one contiguous record per row instead of seven scattered ones:
 //   [cam 3 | quat 4 | scale 3 | opacity | plane index (int bits) | colour C | phase C]
-// The backward packs the M output-gradient rows the same way, in depth order:
-//   [cam 3 (+ z) | quat 4 | scale 3 | opacity | colour C | phase C | plane P]
-// and a second pass in parameter order reads its row's record.
+// The backward packs the M output-gradient rows the same way,
+//   [cam 3 (+ z) | quat 4 | scale 3 | opacity | colour C | phase C | plane P],
+// each at its parameter row, and a second pass reads them in parameter order.
 __host__ __device__ constexpr int round4(int x) { return (x + 3) & ~3; }
 __host__ __device__ constexpr int fwd_stride(int C) { return round4(12 + 2 * C); }
 __host__ __device__ constexpr int bwd_stride(int C, int P) { return round4(11 + 2 * C + P); }
 
-constexpr uint32_t kNotSelected = 0xFFFFFFFFu;
-
-// Registers of one record when its stride is a compile-time constant (kS > 0):
-// filled or drained with 16-byte accesses; with kS == 0 every element goes
-// straight to or from memory.
+// One record per thread.  With a compile-time stride (kS > 0) the block's
+// records pass through LDS, so that kS / 4 neighbouring lanes move one
+// record's 16-byte pieces and a record costs memory one or two requests, not
+// one per piece and lane (the backward's scattered stores: 80 -> 65 us at 1M
+// rows of 80 bytes); with kS == 0 every element goes straight to or from
+// memory.
 template <int kS>
 struct Rec {
+  static constexpr int kPieces = kS > 0 ? kS / 4 : 1;
   float v[kS > 0 ? kS : 1] = {};
-  float* mem;
-  __device__ __forceinline__ explicit Rec(float* p) : mem(p) {}
+  float* mem = nullptr;  // kS == 0: this thread's record
   __device__ __forceinline__ void put(int k, float x) {
     if constexpr (kS > 0) v[k] = x; else mem[k] = x;
   }
   __device__ __forceinline__ float get(int k) const {
     if constexpr (kS > 0) return v[k]; else return mem[k];
   }
-  __device__ __forceinline__ void store() {
+  // The whole block, after put(): thread i's record goes to base + row_i
+  // stride, or nowhere with row_i < 0.
+  __device__ __forceinline__ void store(float* base, int64_t row, float4* s_rec, int64_t* s_row) {
     if constexpr (kS > 0) {
 #pragma unroll
-      for (int k = 0; k < kS; k += 4)
-        *reinterpret_cast<float4*>(mem + k) = make_float4(v[k], v[k + 1], v[k + 2], v[k + 3]);
+      for (int k = 0; k < kPieces; ++k)
+        s_rec[threadIdx.x * kPieces + k] =
+            make_float4(v[4 * k], v[4 * k + 1], v[4 * k + 2], v[4 * k + 3]);
+      s_row[threadIdx.x] = row;
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < kPieces; ++k) {
+        const int i = threadIdx.x + k * kPreThreads;
+        const int64_t r = s_row[i / kPieces];
+        if (r >= 0) reinterpret_cast<float4*>(base)[r * kPieces + i % kPieces] = s_rec[i];
+      }
     }
   }
-  __device__ __forceinline__ void load() {
+  // The whole block, before get(): the reverse.
+  __device__ __forceinline__ void load(const float* base, int64_t row, float4* s_rec,
+                                       int64_t* s_row) {
     if constexpr (kS > 0) {
+      s_row[threadIdx.x] = row;
+      __syncthreads();
 #pragma unroll
-      for (int k = 0; k < kS; k += 4) {
-        const float4 q = *reinterpret_cast<const float4*>(mem + k);
-        v[k] = q.x;
-        v[k + 1] = q.y;
-        v[k + 2] = q.z;
-        v[k + 3] = q.w;
+      for (int k = 0; k < kPieces; ++k) {
+        const int i = threadIdx.x + k * kPreThreads;
+        const int64_t r = s_row[i / kPieces];
+        if (r >= 0) s_rec[i] = reinterpret_cast<const float4*>(base)[r * kPieces + i % kPieces];
+      }
+      __syncthreads();
+#pragma unroll
+      for (int k = 0; k < kPieces; ++k) {
+        const float4 q = s_rec[threadIdx.x * kPieces + k];
+        v[4 * k] = q.x;
+        v[4 * k + 1] = q.y;
+        v[4 * k + 2] = q.z;
+        v[4 * k + 3] = q.w;
       }
     }
   }
 };
+#define HRF_REC_LDS(R)                                               \
+  __shared__ float4 s_rec[kPreThreads * R::kPieces];                 \
+  __shared__ int64_t s_row[kPreThreads]
 
 // torch.remainder(x, 2*pi) with the divisor as float32: fmod (exact), then
 // the sign of the divisor (model.py:602).
@@ -108,69 +145,70 @@ __device__ __forceinline__ float remainder_2pi(float x) {
 
 __device__ __forceinline__ float sigmoidf_(float x) { return 1.0f / (1.0f + expf(-x)); }
 
-// Selection flag and depth sort key of every Gaussian: kept when
-// near < z < far (model.py:1382-1385) and z >= 0 (model.py:1123); the key
-// orders non-negative floats (-0 counts as 0).  A kept Gaussian's record
+// Depth sort key of every Gaussian, and the count of the kept ones per block:
+// kept when near < z < far (model.py:1382-1385) and z >= 0 (model.py:1123);
+// the key orders non-negative floats (-0 counts as 0), less key_base, and is
+// key_drop, above every kept one, for a dropped row.  A kept Gaussian's record
 // carries its activations (model.py:594-608): F.normalize(q) with eps 1e-12,
 // exp(log-scales), sigmoid(opacity), colours, phase mod 2*pi and the
 // argmax plane (first maximal entry, NaN counting as the maximum).
 template <int kC>
 __global__ __launch_bounds__(kPreThreads) void k_pre_select(
     hrf_scene_params sp, const float* __restrict__ R, const float* __restrict__ T,
-    float near_plane, float far_plane, uint32_t* __restrict__ flag, uint32_t* __restrict__ key,
+    float near_plane, float far_plane, uint32_t key_base, uint32_t key_drop,
+    uint32_t* __restrict__ key, uint64_t* __restrict__ part_t, uint32_t* __restrict__ part_v,
     float* __restrict__ rec) {
   const int64_t g = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (g >= sp.n) return;
-  const View v = load_view(R, T);
-  float c[3];
-  to_camera(v, sp.means[3 * g], sp.means[3 * g + 1], sp.means[3 * g + 2], c);
-  const float z = c[2];
-  const bool keep = z > near_plane && z < far_plane && z >= 0.0f;
-  flag[g] = keep ? 1u : 0u;
-  key[g] = __float_as_uint(z) & 0x7FFFFFFFu;
-  if (!keep) return;
+  float c[3] = {0.0f, 0.0f, 0.0f};
+  bool keep = false;
+  if (g < sp.n) {
+    const View v = load_view(R, T);
+    to_camera(v, sp.means[3 * g], sp.means[3 * g + 1], sp.means[3 * g + 2], c);
+    const float z = c[2];
+    keep = z > near_plane && z < far_plane && z >= 0.0f;
+    key[g] = keep ? (__float_as_uint(z) & 0x7FFFFFFFu) - key_base : key_drop;
+  }
+  const int kept = __syncthreads_count(keep ? 1 : 0);
+  if (threadIdx.x == 0) {
+    part_t[blockIdx.x] = static_cast<uint64_t>(kept);
+    part_v[blockIdx.x] = static_cast<uint32_t>(kept);
+  }
   const int C = kC > 0 ? kC : sp.channels, P = sp.planes;
-  Rec<(kC > 0 ? fwd_stride(kC) : 0)> r(rec + g * fwd_stride(C));
-  r.put(0, c[0]);
-  r.put(1, c[1]);
-  r.put(2, c[2]);
-  const float q0 = sp.pre_quats[4 * g], q1 = sp.pre_quats[4 * g + 1];
-  const float q2 = sp.pre_quats[4 * g + 2], q3 = sp.pre_quats[4 * g + 3];
-  const float nrm = fmaxf(sqrtf(q0 * q0 + q1 * q1 + q2 * q2 + q3 * q3), 1e-12f);
-  r.put(3, q0 / nrm);
-  r.put(4, q1 / nrm);
-  r.put(5, q2 / nrm);
-  r.put(6, q3 / nrm);
+  using R_ = Rec<(kC > 0 ? fwd_stride(kC) : 0)>;
+  HRF_REC_LDS(R_);
+  R_ r;
+  r.mem = rec + g * fwd_stride(C);
+  if (keep) {
+    r.put(0, c[0]);
+    r.put(1, c[1]);
+    r.put(2, c[2]);
+    const float q0 = sp.pre_quats[4 * g], q1 = sp.pre_quats[4 * g + 1];
+    const float q2 = sp.pre_quats[4 * g + 2], q3 = sp.pre_quats[4 * g + 3];
+    const float nrm = fmaxf(sqrtf(q0 * q0 + q1 * q1 + q2 * q2 + q3 * q3), 1e-12f);
+    r.put(3, q0 / nrm);
+    r.put(4, q1 / nrm);
+    r.put(5, q2 / nrm);
+    r.put(6, q3 / nrm);
 #pragma unroll
-  for (int j = 0; j < 3; ++j) r.put(7 + j, expf(sp.pre_scales[3 * g + j]));
-  r.put(10, sigmoidf_(sp.pre_opacities[g]));
-  int best = 0;
-  float bv = sp.pre_plane[g * P];
-  for (int p = 1; p < P; ++p) {
-    const float x = sp.pre_plane[g * P + p];
-    if (!(bv != bv) && (x > bv || x != x)) {
-      bv = x;
-      best = p;
+    for (int j = 0; j < 3; ++j) r.put(7 + j, expf(sp.pre_scales[3 * g + j]));
+    r.put(10, sigmoidf_(sp.pre_opacities[g]));
+    int best = 0;
+    float bv = sp.pre_plane[g * P];
+    for (int p = 1; p < P; ++p) {
+      const float x = sp.pre_plane[g * P + p];
+      if (!(bv != bv) && (x > bv || x != x)) {
+        bv = x;
+        best = p;
+      }
+    }
+    r.put(11, __int_as_float(best));
+#pragma unroll
+    for (int j = 0; j < C; ++j) {
+      r.put(12 + j, sp.colours[g * C + j]);
+      r.put(12 + C + j, remainder_2pi(sp.pre_phase[g * C + j]));
     }
   }
-  r.put(11, __int_as_float(best));
-#pragma unroll
-  for (int j = 0; j < C; ++j) {
-    r.put(12 + j, sp.colours[g * C + j]);
-    r.put(12 + C + j, remainder_2pi(sp.pre_phase[g * C + j]));
-  }
-  r.store();
-}
-
-__global__ __launch_bounds__(kPreThreads) void k_pre_compact(
-    const uint32_t* __restrict__ flag, const uint32_t* __restrict__ pos,
-    const uint32_t* __restrict__ key, int64_t n, uint32_t* __restrict__ ckey,
-    uint32_t* __restrict__ cidx) {
-  const int64_t g = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (g >= n || !flag[g]) return;
-  const uint32_t p = pos[g];
-  ckey[p] = key[g];
-  cidx[p] = static_cast<uint32_t>(g);
+  r.store(rec, keep ? g : -1, s_rec, s_row);
 }
 
 // The m selected Gaussians in depth order: one record read per row, the
@@ -182,11 +220,14 @@ __global__ __launch_bounds__(kPreThreads) void k_pre_gather(
     float* __restrict__ scales, float* __restrict__ colours, float* __restrict__ phase,
     float* __restrict__ opac, float* __restrict__ pprobs, int64_t* __restrict__ idxs) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  const int64_t g = sidx[i];
+  const int64_t g = i < m ? static_cast<int64_t>(sidx[i]) : -1;
   const int C = kC > 0 ? kC : channels;
-  Rec<(kC > 0 ? fwd_stride(kC) : 0)> r(const_cast<float*>(rec) + g * fwd_stride(C));
-  r.load();
+  using R_ = Rec<(kC > 0 ? fwd_stride(kC) : 0)>;
+  HRF_REC_LDS(R_);
+  R_ r;
+  r.mem = const_cast<float*>(rec) + g * fwd_stride(C);
+  r.load(rec, g, s_rec, s_row);
+  if (i >= m) return;
 #pragma unroll
   for (int j = 0; j < 3; ++j) cam[3 * i + j] = r.get(j);
   zv[i] = r.get(2);
@@ -206,34 +247,40 @@ __global__ __launch_bounds__(kPreThreads) void k_pre_gather(
 }
 
 // Backward, pass 1 (depth order): pack the output-gradient rows of each
-// selected Gaussian and record its position under its parameter row.
+// selected Gaussian into its parameter row's record and mark the row.  (An
+// inverse permutation and records in depth order cost a random 4-byte store
+// here and random records in pass 2: 60 + 72 us at 1M rows, against 65 + 50.)
 template <int kC, int kP>
 __global__ __launch_bounds__(kPreThreads) void k_pre_bpack(
     const int64_t* __restrict__ idxs, int64_t m, int64_t n, int channels, int planes,
-    hrf_selected_grads gin, float* __restrict__ grec, uint32_t* __restrict__ inv) {
+    hrf_selected_grads gin, float* __restrict__ grec, uint8_t* __restrict__ mark) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= m) return;
-  const int64_t g = idxs[i];
-  if (g < 0 || g >= n) return;
+  int64_t g = i < m ? idxs[i] : -1;
+  if (g >= n) g = -1;
   const int C = kC > 0 ? kC : channels, P = kP > 0 ? kP : planes;
-  Rec<(kC > 0 && kP > 0 ? bwd_stride(kC, kP) : 0)> r(grec + i * bwd_stride(C, P));
-  r.put(0, gin.cam[3 * i]);
-  r.put(1, gin.cam[3 * i + 1]);
-  r.put(2, gin.cam[3 * i + 2] + (gin.z ? gin.z[i] : 0.0f));
+  using R_ = Rec<(kC > 0 && kP > 0 ? bwd_stride(kC, kP) : 0)>;
+  HRF_REC_LDS(R_);
+  R_ r;
+  r.mem = grec + g * bwd_stride(C, P);
+  if (g >= 0) {
+    r.put(0, gin.cam[3 * i]);
+    r.put(1, gin.cam[3 * i + 1]);
+    r.put(2, gin.cam[3 * i + 2] + (gin.z ? gin.z[i] : 0.0f));
 #pragma unroll
-  for (int j = 0; j < 4; ++j) r.put(3 + j, gin.quats[4 * i + j]);
+    for (int j = 0; j < 4; ++j) r.put(3 + j, gin.quats[4 * i + j]);
 #pragma unroll
-  for (int j = 0; j < 3; ++j) r.put(7 + j, gin.scales[3 * i + j]);
-  r.put(10, gin.opacities[i]);
+    for (int j = 0; j < 3; ++j) r.put(7 + j, gin.scales[3 * i + j]);
+    r.put(10, gin.opacities[i]);
 #pragma unroll
-  for (int j = 0; j < C; ++j) {
-    r.put(11 + j, gin.colours[i * C + j]);
-    r.put(11 + C + j, gin.phase[i * C + j]);
+    for (int j = 0; j < C; ++j) {
+      r.put(11 + j, gin.colours[i * C + j]);
+      r.put(11 + C + j, gin.phase[i * C + j]);
+    }
+#pragma unroll
+    for (int p = 0; p < P; ++p) r.put(11 + 2 * C + p, gin.plane_probs[i * P + p]);
+    mark[g] = 1;
   }
-#pragma unroll
-  for (int p = 0; p < P; ++p) r.put(11 + 2 * C + p, gin.plane_probs[i * P + p]);
-  r.store();
-  inv[g] = static_cast<uint32_t>(i);
+  r.store(grec, g, s_rec, s_row);
 }
 
 // Backward, pass 2 (parameter order): every parameter-gradient row, zero for
@@ -244,13 +291,18 @@ __global__ __launch_bounds__(kPreThreads) void k_pre_bpack(
 // (model.py:50-56).
 template <int kC, int kP>
 __global__ __launch_bounds__(kPreThreads) void k_pre_bscatter(
-    hrf_scene_params sp, const float* __restrict__ R, const uint32_t* __restrict__ inv,
+    hrf_scene_params sp, const float* __restrict__ R, const uint8_t* __restrict__ mark,
     const float* __restrict__ grec, hrf_param_grads d) {
   const int64_t g = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (g >= sp.n) return;
   const int C = kC > 0 ? kC : sp.channels, P = kP > 0 ? kP : sp.planes;
-  const uint32_t i = inv[g];
-  if (i == kNotSelected) {
+  const bool selected = g < sp.n && mark[g] != 0;
+  using R_ = Rec<(kC > 0 && kP > 0 ? bwd_stride(kC, kP) : 0)>;
+  HRF_REC_LDS(R_);
+  R_ r;
+  r.mem = const_cast<float*>(grec) + g * bwd_stride(C, P);
+  r.load(grec, selected ? g : -1, s_rec, s_row);
+  if (g >= sp.n) return;
+  if (!selected) {
 #pragma unroll
     for (int j = 0; j < 3; ++j) {
       d.means[3 * g + j] = 0.0f;
@@ -268,9 +320,6 @@ __global__ __launch_bounds__(kPreThreads) void k_pre_bscatter(
     for (int p = 0; p < P; ++p) d.pre_plane[g * P + p] = 0.0f;
     return;
   }
-  Rec<(kC > 0 && kP > 0 ? bwd_stride(kC, kP) : 0)> r(
-      const_cast<float*>(grec) + static_cast<int64_t>(i) * bwd_stride(C, P));
-  r.load();
   const float gc0 = r.get(0), gc1 = r.get(1), gc2 = r.get(2);
 #pragma unroll
   for (int k = 0; k < 3; ++k)
@@ -312,17 +361,13 @@ __global__ __launch_bounds__(kPreThreads) void k_pre_bscatter(
 }
 
 struct PreWs {
-  uint32_t* flag;
-  uint32_t* pos;
   uint32_t* key;
-  uint32_t* ckey;
-  uint32_t* cidx;
-  uint32_t* ckey_b;
-  uint32_t* cidx_b;
-  uint64_t* off;
-  uint64_t* bsum_p;
-  uint32_t* bsum_v;
-  uint32_t* zero;
+  uint32_t* key_b;
+  uint32_t* idx;  // the sort ends here
+  uint32_t* idx_b;
+  uint64_t* part_t;  // per-block counts of kept rows, in both of the scan's forms
+  uint32_t* part_v;
+  uint32_t* scan_flag;
   uint32_t* radix;
   float* rec;  // n records of fwd_stride(C) floats, written for kept rows
 };
@@ -330,34 +375,32 @@ struct PreWs {
 PreWs carve_pre(Carver& cv, int64_t n, int C) {
   PreWs w;
   const int64_t m = n > 0 ? n : 1;
-  w.flag = cv.take<uint32_t>(m);
-  w.pos = cv.take<uint32_t>(m);
   w.key = cv.take<uint32_t>(m);
-  w.ckey = cv.take<uint32_t>(m);
-  w.cidx = cv.take<uint32_t>(m);
-  w.ckey_b = cv.take<uint32_t>(m);
-  w.cidx_b = cv.take<uint32_t>(m);
-  w.off = cv.take<uint64_t>(m + 1);
-  w.bsum_p = cv.take<uint64_t>(scan_scratch_elems(m));
-  w.bsum_v = cv.take<uint32_t>(scan_scratch_elems(m));
-  w.zero = cv.take<uint32_t>(4);
+  w.key_b = cv.take<uint32_t>(m);
+  w.idx = cv.take<uint32_t>(m);
+  w.idx_b = cv.take<uint32_t>(m);
+  w.part_t = cv.take<uint64_t>(partial_elems(m));
+  w.part_v = cv.take<uint32_t>(partial_elems(m));
+  w.scan_flag = cv.take<uint32_t>(4);
   w.radix = cv.take<uint32_t>(radix_scratch_elems(m));
   w.rec = cv.take<float>(m * fwd_stride(C));
   return w;
 }
 
 // The backward's layout of the same workspace (nothing carries over from
-// the forward): the position of each parameter row in depth order
-// (kNotSelected if it was not selected) and the packed gradient records.
+// the forward): one byte per parameter row, set where it was selected, and
+// the packed gradient records.
 struct PreBwdWs {
-  uint32_t* inv;
+  uint32_t* mark;  // n bytes, cleared as words
   float* grec;
 };
+
+int64_t mark_words(int64_t n) { return (n + 3) / 4; }
 
 PreBwdWs carve_pre_bwd(Carver& cv, int64_t n, int C, int P) {
   PreBwdWs w;
   const int64_t m = n > 0 ? n : 1;
-  w.inv = cv.take<uint32_t>(m);
+  w.mark = cv.take<uint32_t>(mark_words(m));
   w.grec = cv.take<float>(m * bwd_stride(C, P));
   return w;
 }
@@ -385,6 +428,26 @@ int check_params(const hrf_scene_params* sp) {
               static_cast<long long>(sp->n));
     return HRF_ERR_INVALID;
   }
+  return HRF_OK;
+}
+
+// The backward's two passes.  kC, kP > 0: records of compile-time size, in
+// registers between 16-byte accesses (2.6M rows of six planes: 948 us with the
+// run-time size and an inverse permutation, 342 us with this); the general form
+// moves every element by itself.
+template <int kC, int kP>
+int pre_backward(const hrf_scene_params* sp, const float* R, const int64_t* idxs, int64_t m,
+                 const hrf_selected_grads* grads, const hrf_param_grads* out, float* grec,
+                 uint8_t* mark, hipStream_t s) {
+  if (m > 0) {
+    hipLaunchKernelGGL((k_pre_bpack<kC, kP>), dim3(blocks_for(m, kPreThreads)),
+                       dim3(kPreThreads), 0, s, idxs, m, sp->n, sp->channels, sp->planes, *grads,
+                       grec, mark);
+    HRF_LAUNCH_CHECK();
+  }
+  hipLaunchKernelGGL((k_pre_bscatter<kC, kP>), dim3(blocks_for(sp->n, kPreThreads)),
+                     dim3(kPreThreads), 0, s, *sp, R, mark, grec, *out);
+  HRF_LAUNCH_CHECK();
   return HRF_OK;
 }
 
@@ -423,24 +486,40 @@ int hrf_preprocess_select(const hrf_scene_params* sp, const float* R, const floa
   HRF_TRY(readback_acquire(&slot.r));
   const uint64_t tag = readback_arm(slot.r);
   HRF_STAGE("pre_select", s);
-  HRF_TRY(launch_fill_u32(w.zero, 0u, 1, s));
   const dim3 grid(blocks_for(n, kPreThreads));
+  // Keys of depths in (max(near, 0), far): see the head of this file.
+  const float lo = near_plane > 0.0f ? near_plane : 0.0f;
+  uint32_t key_base, key_drop;
+  std::memcpy(&key_base, &lo, sizeof(key_base));
+  std::memcpy(&key_drop, &far_plane, sizeof(key_drop));
+  key_drop = far_plane > lo ? key_drop - key_base : 1u;  // else nothing is kept
+  int key_bits = 1;
+  while (key_bits < 32 && key_drop >> key_bits) ++key_bits;
   if (sp->channels == 3)
     hipLaunchKernelGGL(k_pre_select<3>, grid, dim3(kPreThreads), 0, s, *sp, R, T, near_plane,
-                       far_plane, w.flag, w.key, w.rec);
+                       far_plane, key_base, key_drop, w.key, w.part_t, w.part_v, w.rec);
   else
     hipLaunchKernelGGL(k_pre_select<0>, grid, dim3(kPreThreads), 0, s, *sp, R, T, near_plane,
-                       far_plane, w.flag, w.key, w.rec);
+                       far_plane, key_base, key_drop, w.key, w.part_t, w.part_v, w.rec);
   HRF_LAUNCH_CHECK();
-  // Exclusive positions of the kept Gaussians (the binning's offsets scan,
-  // with the flags as both of its inputs); totals[1] = kept count, written
-  // into the pinned read-back words, read while the compaction runs.
+  // totals[1] = kept count, written into the pinned read-back words and read
+  // while the sort runs.
+  static_assert(kPreThreads == kProjThreads, "one count per block of the scan");
   slot.pending = true;
-  HRF_TRY(launch_offsets(nullptr, w.flag, w.flag, n, w.off, w.pos, w.bsum_p, w.bsum_v, w.zero,
-                         slot.r->dev, s, tag));
-  hipLaunchKernelGGL(k_pre_compact, grid, dim3(kPreThreads), 0, s, w.flag, w.pos, w.key, n,
-                     w.ckey, w.cidx);
-  HRF_LAUNCH_CHECK();
+  HRF_TRY(launch_partials_scan(w.part_t, w.part_v, n, w.scan_flag, slot.r->dev, s, tag));
+  if (n > 1) {
+    // Stable ascending depth order (ties keep index order), ending in w.idx.
+    const bool odd = radix_passes(key_bits) % 2 == 1;
+    bool in_b = false;
+    HRF_TRY(radix_sort_pairs(w.key, odd ? w.idx_b : w.idx, w.key_b, odd ? w.idx : w.idx_b, n,
+                             key_bits, w.radix, &in_b, s, nullptr, true, false));
+    if (in_b != odd) {
+      set_error("internal: preprocess sort ended in the wrong buffer");
+      return HRF_ERR_INVALID;
+    }
+  } else {
+    HRF_TRY(launch_fill_u32(w.idx, 0u, 1, s));
+  }
   HRF_TRY(readback_wait(slot.r, tag, s));
   slot.pending = false;
   const uint64_t kept = slot.r->host[1];
@@ -450,16 +529,6 @@ int hrf_preprocess_select(const hrf_scene_params* sp, const float* R, const floa
     return HRF_ERR_INVALID;
   }
   const int64_t m = static_cast<int64_t>(kept);
-  if (m > 1) {
-    // Stable ascending depth order (ties keep index order); 4 passes, so
-    // the result ends in (ckey, cidx).
-    bool in_b = false;
-    HRF_TRY(radix_sort_pairs(w.ckey, w.cidx, w.ckey_b, w.cidx_b, m, 32, w.radix, &in_b, s));
-    if (in_b) {
-      set_error("internal: preprocess sort expected an even pass count");
-      return HRF_ERR_INVALID;
-    }
-  }
   *num_selected = m;
   return HRF_OK;
 }
@@ -493,11 +562,11 @@ int hrf_preprocess_forward(const hrf_scene_params* sp, const float* R, const flo
   const dim3 grid(blocks_for(m, kPreThreads));
   if (sp->channels == 3)
     hipLaunchKernelGGL(k_pre_gather<3>, grid, dim3(kPreThreads), 0, s, w.rec, sp->channels,
-                       sp->planes, w.cidx, m, cam_means, z_vals, quats, scales, colours, phase,
+                       sp->planes, w.idx, m, cam_means, z_vals, quats, scales, colours, phase,
                        opacities, plane_probs, idxs);
   else
     hipLaunchKernelGGL(k_pre_gather<0>, grid, dim3(kPreThreads), 0, s, w.rec, sp->channels,
-                       sp->planes, w.cidx, m, cam_means, z_vals, quats, scales, colours, phase,
+                       sp->planes, w.idx, m, cam_means, z_vals, quats, scales, colours, phase,
                        opacities, plane_probs, idxs);
   HRF_LAUNCH_CHECK();
   return HRF_OK;
@@ -533,28 +602,20 @@ int hrf_preprocess_backward(const hrf_scene_params* sp, const float* R, const in
   hipStream_t s = static_cast<hipStream_t>(stream);
   Carver cv(ws);
   PreBwdWs w = carve_pre_bwd(cv, n, sp->channels, sp->planes);
-  const bool fast = sp->channels == 3 && sp->planes == 3;
   HRF_STAGE("pre_backward", s);
-  HRF_TRY(launch_fill_u32(w.inv, kNotSelected, n, s));
-  if (m > 0) {
-    const dim3 grid(blocks_for(m, kPreThreads));
-    if (fast)
-      hipLaunchKernelGGL((k_pre_bpack<3, 3>), grid, dim3(kPreThreads), 0, s, idxs, m, n,
-                         sp->channels, sp->planes, *grads, w.grec, w.inv);
-    else
-      hipLaunchKernelGGL((k_pre_bpack<0, 0>), grid, dim3(kPreThreads), 0, s, idxs, m, n,
-                         sp->channels, sp->planes, *grads, w.grec, w.inv);
-    HRF_LAUNCH_CHECK();
+  HRF_TRY(launch_fill_u32(w.mark, 0u, mark_words(n), s));
+  uint8_t* mark = reinterpret_cast<uint8_t*>(w.mark);
+  if (sp->channels == 3 && sp->planes <= 6) {
+    switch (sp->planes) {
+      case 1: return pre_backward<3, 1>(sp, R, idxs, m, grads, out, w.grec, mark, s);
+      case 2: return pre_backward<3, 2>(sp, R, idxs, m, grads, out, w.grec, mark, s);
+      case 3: return pre_backward<3, 3>(sp, R, idxs, m, grads, out, w.grec, mark, s);
+      case 4: return pre_backward<3, 4>(sp, R, idxs, m, grads, out, w.grec, mark, s);
+      case 5: return pre_backward<3, 5>(sp, R, idxs, m, grads, out, w.grec, mark, s);
+      default: return pre_backward<3, 6>(sp, R, idxs, m, grads, out, w.grec, mark, s);
+    }
   }
-  const dim3 grid(blocks_for(n, kPreThreads));
-  if (fast)
-    hipLaunchKernelGGL((k_pre_bscatter<3, 3>), grid, dim3(kPreThreads), 0, s, *sp, R, w.inv,
-                       w.grec, *out);
-  else
-    hipLaunchKernelGGL((k_pre_bscatter<0, 0>), grid, dim3(kPreThreads), 0, s, *sp, R, w.inv,
-                       w.grec, *out);
-  HRF_LAUNCH_CHECK();
-  return HRF_OK;
+  return pre_backward<0, 0>(sp, R, idxs, m, grads, out, w.grec, mark, s);
 }
 
 }  // extern "C"

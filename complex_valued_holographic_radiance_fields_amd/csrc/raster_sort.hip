@@ -17,10 +17,6 @@
 namespace hrf {
 namespace {
 
-constexpr int kScanThreads = 256;
-constexpr int kScanItems = 8;
-constexpr int kScanTile = kScanThreads * kScanItems;  // elements per block
-
 constexpr int kRadixItems = 8;  // keys per thread and tile
 // Block size of the radix kernels: 256 threads (2048-key tiles), or 1024
 // (8192-key tiles) for sorts of at least kRadixLargeMinKeys keys.  Longer
@@ -502,73 +498,9 @@ __device__ __forceinline__ uint32_t ordered(const uint32_t* order, const uint32_
   return *sorted_flag ? order[i] : static_cast<uint32_t>(i);
 }
 
-// Pair and visible offsets (three launches for both scans).  Pair counts
-// are taken in depth-rank order (tiles[order[i]], or tiles[i] with no
-// order), visibility flags in index order.
-//   k_offsets_reduce: per-block sums of both arrays;
-//   k_offsets_blocks: one block scans the block sums in place (exclusive) and
-//     writes the totals [K, V, *sort_flag] and off[n] = K;
-//   k_offsets_scan: per-block exclusive scans plus the block prefixes.
-__device__ __forceinline__ void load_counts(const uint32_t* __restrict__ order,
-                                            const uint32_t* __restrict__ tiles,
-                                            const uint32_t* __restrict__ vis, int64_t n,
-                                            int64_t base, uint32_t (&t)[kScanItems],
-                                            uint32_t (&v)[kScanItems]) {
-#pragma unroll
-  for (int i = 0; i < kScanItems; ++i) {
-    const int64_t idx = base + i;
-    t[i] = 0u;
-    v[i] = 0u;
-    if (idx < n) {
-      t[i] = tiles[order ? order[idx] : static_cast<uint32_t>(idx)];
-      v[i] = vis[idx];
-    }
-  }
-}
-
-__global__ __launch_bounds__(kScanThreads) void k_offsets_reduce(
-    const uint32_t* __restrict__ order, const uint32_t* __restrict__ tiles,
-    const uint32_t* __restrict__ vis, int64_t n, uint64_t* __restrict__ bsum_p,
-    uint32_t* __restrict__ bsum_v) {
-  __shared__ uint64_t s_p[kScanThreads / 64];
-  __shared__ uint32_t s_v[kScanThreads / 64];
-  uint32_t t[kScanItems], v[kScanItems];
-  load_counts(order, tiles, vis, n,
-              static_cast<int64_t>(blockIdx.x) * kScanTile +
-                  static_cast<int64_t>(threadIdx.x) * kScanItems,
-              t, v);
-  uint64_t sp = 0;
-  uint32_t sv = 0;
-#pragma unroll
-  for (int i = 0; i < kScanItems; ++i) {
-    sp += t[i];
-    sv += v[i];
-  }
-#pragma unroll
-  for (int d = 32; d >= 1; d >>= 1) {
-    sp += __shfl_xor(sp, d, 64);
-    sv += __shfl_xor(sv, d, 64);
-  }
-  const int wave = threadIdx.x >> 6;
-  if ((threadIdx.x & 63) == 0) {
-    s_p[wave] = sp;
-    s_v[wave] = sv;
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    uint64_t a = 0;
-    uint32_t b = 0;
-#pragma unroll
-    for (int w = 0; w < kScanThreads / 64; ++w) {
-      a += s_p[w];
-      b += s_v[w];
-    }
-    bsum_p[blockIdx.x] = a;
-    bsum_v[blockIdx.x] = b;
-  }
-}
-
-template <int THREADS = kScanThreads, int ITEMS = kScanItems>
+// One block scans per-block sums of the pair and visible counts in place
+// (exclusive) and writes the totals [K, V, *sort_flag] and off_end[0] = K.
+template <int THREADS, int ITEMS>
 __global__ __launch_bounds__(THREADS) void k_offsets_blocks(
     uint64_t* __restrict__ bsum_p, uint32_t* __restrict__ bsum_v, int64_t nb,
     uint64_t* __restrict__ off_end, const uint32_t* __restrict__ sort_flag,
@@ -673,42 +605,6 @@ __device__ __forceinline__ void block_offsets(const uint64_t* __restrict__ part_
   const uint64_t b0 = base[blockIdx.x];
   if (static_cast<int>(threadIdx.x) < nr) s_off[threadIdx.x] = b0 + ex;
   if (threadIdx.x == 0) s_off[nr] = b0 + total;
-}
-
-__global__ __launch_bounds__(kScanThreads) void k_offsets_scan(
-    const uint32_t* __restrict__ order, const uint32_t* __restrict__ tiles,
-    const uint32_t* __restrict__ vis, int64_t n, const uint64_t* __restrict__ bsum_p,
-    const uint32_t* __restrict__ bsum_v, uint64_t* __restrict__ off,
-    uint32_t* __restrict__ vis_off) {
-  __shared__ uint64_t s_wp[kScanThreads / 64];
-  __shared__ uint32_t s_wv[kScanThreads / 64];
-  const int64_t base = static_cast<int64_t>(blockIdx.x) * kScanTile +
-                       static_cast<int64_t>(threadIdx.x) * kScanItems;
-  uint32_t t[kScanItems], v[kScanItems];
-  load_counts(order, tiles, vis, n, base, t, v);
-  uint64_t p[kScanItems];
-  uint32_t q[kScanItems];
-  uint64_t rp = 0;
-  uint32_t rv = 0;
-#pragma unroll
-  for (int i = 0; i < kScanItems; ++i) {
-    p[i] = rp;
-    q[i] = rv;
-    rp += t[i];
-    rv += v[i];
-  }
-  uint64_t tp;
-  uint32_t tv;
-  const uint64_t op = block_exclusive_scan<uint64_t>(rp, &tp, s_wp) + bsum_p[blockIdx.x];
-  const uint32_t ov = block_exclusive_scan<uint32_t>(rv, &tv, s_wv) + bsum_v[blockIdx.x];
-#pragma unroll
-  for (int i = 0; i < kScanItems; ++i) {
-    const int64_t idx = base + i;
-    if (idx < n) {
-      off[idx] = op + p[i];
-      vis_off[idx] = ov + q[i];
-    }
-  }
 }
 
 // Pairs [a, a + cnt) of an emission block, whose pair offsets are
@@ -1230,17 +1126,6 @@ __global__ __launch_bounds__(kDiffThreads) void k_ranges_from_diff(const int32_t
 
 }  // namespace
 
-size_t scan_scratch_elems(int64_t n) {
-  size_t total = 0;
-  int64_t m = n;
-  while (m > 1) {
-    m = (m + kScanTile - 1) / kScanTile;
-    total += static_cast<size_t>(m);
-  }
-  return total + 4;
-}
-
-
 int radix_passes(int end_bit) { return (end_bit + 7) / 8; }
 
 size_t radix_scratch_elems(int64_t n) {
@@ -1509,24 +1394,6 @@ int launch_fill_f32(float* p, float v, int64_t n, hipStream_t s) {
                        n - head);
     HRF_LAUNCH_CHECK();
   }
-  return HRF_OK;
-}
-
-int launch_offsets(const uint32_t* order, const uint32_t* tiles, const uint32_t* vis,
-                   int64_t n, uint64_t* off, uint32_t* vis_off, uint64_t* bsum_p,
-                   uint32_t* bsum_v, const uint32_t* sort_flag, uint64_t* totals,
-                   hipStream_t s, uint64_t tag) {
-  if (n <= 0) return HRF_OK;
-  const int64_t nb = (n + kScanTile - 1) / kScanTile;
-  hipLaunchKernelGGL(k_offsets_reduce, dim3(static_cast<unsigned>(nb)), dim3(kScanThreads), 0,
-                     s, order, tiles, vis, n, bsum_p, bsum_v);
-  HRF_LAUNCH_CHECK();
-  hipLaunchKernelGGL((k_offsets_blocks<>), dim3(1), dim3(kScanThreads), 0, s, bsum_p, bsum_v,
-                     nb, off + n, sort_flag, totals, nullptr, tag);
-  HRF_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_offsets_scan, dim3(static_cast<unsigned>(nb)), dim3(kScanThreads), 0, s,
-                     order, tiles, vis, n, bsum_p, bsum_v, off, vis_off);
-  HRF_LAUNCH_CHECK();
   return HRF_OK;
 }
 

@@ -1,0 +1,79 @@
+"""The preprocess at the edges of its depth keys (their width sets the sort's
+pass count, dropped rows come last) and of its record sizes."""
+import numpy as np
+import pytest
+
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+
+def _params(n, P, C, z, seed):
+    rng = np.random.default_rng(seed)
+    means = rng.normal(size=(n, 3)).astype(np.float32)
+    means[:, 2] = z
+    return (means, rng.normal(size=(n, 4)).astype(np.float32),
+            rng.normal(-4, 0.5, size=(n, 3)).astype(np.float32),
+            rng.uniform(size=(n, C)).astype(np.float32),
+            rng.uniform(-20, 20, size=(n, C)).astype(np.float32),
+            rng.normal(size=n).astype(np.float32), rng.normal(size=(n, P)).astype(np.float32),
+            np.eye(3, dtype=np.float32), np.zeros(3, np.float32))
+
+
+def _t(a):
+    import torch
+
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+UP = np.float32(np.nextafter(np.float32(2), np.float32(3)))
+# near, far, depths: key bits and passes in the comment
+RANGES = {
+    "one_bit": (1.9999999, float(UP), [2.0]),                   # the least key above near's
+    "one_pass": (2.0, 2.00003, [2.00001, 2.00002, 2.0, 1.0]),    # 7 bits
+    "three_passes": (2.0, 3.0, None),                            # 22 bits
+    "wide": (1e-30, 1e30, None),                                 # 30 bits
+    "negative_near": (-5.0, 4.0, [0.0, -0.0, -1.0, 1e-42, 3.0, 4.0]),  # z >= 0 holds
+    "infinite_far": (1.0, float("inf"), [3e38, 1.5, float("inf"), float("nan"), 2.0]),
+    "far_below_near": (3.0, 2.0, None),
+    "nothing_positive": (-5.0, -1.0, None),
+}
+
+
+@pytest.mark.parametrize("name", list(RANGES))
+@pytest.mark.parametrize("n", [1, 2, 5000])
+def test_depth_ranges(hrf, oracle_mod, name, n):
+    from complex_valued_holographic_radiance_fields_amd import preprocess
+
+    near, far, depths = RANGES[name]
+    rng = np.random.default_rng(n)
+    z = rng.uniform(0.5, 4.5, size=n) if depths is None else rng.choice(depths, size=n)
+    prm = _params(n, 3, 3, z.astype(np.float32), n)
+    ref = oracle_mod.preprocess_forward(*prm, near=near, far=far)
+    out = [o.cpu().numpy() for o in preprocess.forward(*[_t(a) for a in prm], near, far)]
+    np.testing.assert_array_equal(out[-1], ref["idxs"])
+    np.testing.assert_array_equal(out[1], ref["z"])
+    np.testing.assert_array_equal(out[0], ref["cam"])
+
+
+@pytest.mark.parametrize("C", [2, 3])
+@pytest.mark.parametrize("P", [1, 2, 3, 4, 5, 6, 7])
+def test_backward_record_sizes(hrf, oracle_mod, P, C):
+    """Records of compile-time (C = 3, P <= 6) and run-time size; float32
+    chain rules of a few products each."""
+    from complex_valued_holographic_radiance_fields_amd import preprocess
+
+    n = 777
+    rng = np.random.default_rng(10 * P + C)
+    prm = _params(n, P, C, rng.uniform(0.5, 5.0, size=n).astype(np.float32), P)
+    ref = oracle_mod.preprocess_forward(*prm, near=1.0, far=4.0)
+    keys = ("cam", "z", "quats", "scales", "colours", "phase", "opacities", "plane_probs")
+    g = {k: rng.normal(size=ref[k].shape).astype(np.float32) for k in keys}
+    exp = oracle_mod.preprocess_backward(g, *prm[:7], prm[7], ref["idxs"])
+    got = preprocess.backward([_t(g[k]) for k in keys], *[_t(a) for a in prm[:7]], _t(prm[7]),
+                              _t(ref["idxs"]))
+    names = ("means", "pre_quats", "pre_scales", "colours", "pre_phase", "pre_opac", "pre_plane")
+    for name, t in zip(names, got):
+        assert rel_l2(t.cpu().numpy(), exp[name]) < 1e-6, name
+        rest = np.setdiff1d(np.arange(n), ref["idxs"])
+        assert not t.cpu().numpy()[rest].any(), name
