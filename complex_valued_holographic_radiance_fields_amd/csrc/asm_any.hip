@@ -9,14 +9,14 @@
 // grid through memory.  Both measured, forward / adjoint, by hipEvents:
 //
 //   fields            grid   library path         these passes
-//   1   (720 x 1280)  2560    229 /  215 us        96 /  92 us
-//   9   (300 x 400)    800    156 /  147 us        69 /  68 us
-//   18  (378 x 504)   1008    379 /  340 us       103 / 105 us
-//   9   (556 x 742)   1484   1195 / 1143 us       397 / 342 us   (chirp)
-//   3   (1424 x 1900) 3800   3000 / 2945 us       887 / 833 us   (chirp)
+//   1   (720 x 1280)  2560    229 /  215 us        93 /  89 us
+//   9   (300 x 400)    800    156 /  147 us        68 /  66 us
+//   18  (378 x 504)   1008    379 /  340 us       101 / 101 us
+//   9   (556 x 742)   1484   1195 / 1143 us       390 / 340 us   (chirp)
+//   3   (1424 x 1900) 3800   3000 / 2945 us       839 / 791 us   (chirp)
 //
 // The column passes are bound by VALU issue and the latency between their
-// barriers (1008 points, 18 fields: 72 us of the 103), the row passes by
+// barriers (1008 points, 18 fields: 66 us of the 101), the row passes by
 // memory latency.
 //
 // Smooth lengths (factors 2, 3, 5, 7): the forward transform is
@@ -77,13 +77,15 @@ struct AnyPlan {
   AnyStage st[kAnyMaxStages];
 };
 
-// LDS layout: transform b of the batch starts at b * line_stride; a half
-// wave's lanes then hold eight consecutive elements of four transforms (16
-// of two) on different banks wherever the span is at least eight.
+// LDS layout: transform b of the batch starts at b * line_stride.  An 8-byte
+// access serves 16 lanes at a time from 32 banks, here 16 / B consecutive
+// elements of B lines wherever the span allows: the stride modulo 16 elements
+// (128 bytes) puts the lines side by side (against a stride modulo 32: a
+// quarter of the bank conflicts, 72 -> 67 us in the 1008-point column pass of 18
+// fields, 324 -> 304 us in the 1484-point chirp one of 9).
 template <int B>
 __host__ __device__ constexpr int line_stride(int n) {
-  constexpr int want = B == 4 ? 8 : 16;  // modulo 32 elements (256 bytes)
-  return n + ((want - n % 32) + 32) % 32;
+  return n + ((16 / B - n % 16) + 16) % 16;
 }
 
 // ---------------------------------------------------------------- stages --
@@ -495,51 +497,6 @@ __global__ __launch_bounds__(768, 4) void k_chirp_rows_out(const float2* __restr
 }
 
 // --------------------------------------------------------- column passes --
-// kz of spectral element (row frequency i, column frequency k), -1 where the
-// evanescent cut or the aperture zeroes the transfer function.
-__device__ __forceinline__ float kz_or_cut(float k0, int i, int k, int M, float sfreq, float ap) {
-  float fx, fy;
-  bool inap, prop;
-  coords(i, k, M, sfreq, ap, &fx, &fy, &inap);
-  const float kk = kz_of(k0, fx, fy, &prop);
-  return prop && inap ? kk : -1.0f;
-}
-
-struct Band {
-  float fxm, fym, d;
-  bool all;
-};
-__device__ __forceinline__ Band band_of(const AsmFftConsts& mc, int p, int c) {
-  return Band{mc.fxmax[p * kMaxChannels + c], mc.fymax[p * kMaxChannels + c], mc.d[p],
-              mc.band_all[p * kMaxChannels + c] != 0};
-}
-// Whether the transfer function passes (i, k), given its kz.
-__device__ __forceinline__ bool passes(const Band& bd, float kz, int i, int k, int M,
-                                       float sfreq) {
-  if (kz < 0.0f) return false;
-  if (bd.all) return true;
-  float fx, fy;
-  bool inap;
-  coords(i, k, M, sfreq, -1.0f, &fx, &fy, &inap);
-  return fabsf(fx) < bd.fxm && fabsf(fy) < bd.fym;
-}
-__device__ __forceinline__ float2 turn(float2 x, float phase) {
-  float sn, cs;
-  sincos_big_ff(phase, &sn, &cs);
-  return make_float2(x.x * cs - x.y * sn, x.x * sn + x.y * cs);
-}
-
-// The block's channel, intermediate tile, first column in it and first
-// spectrum column.
-template <int B>
-__device__ __forceinline__ void column_block(int M, int* c, int* cb, int* col0, int* k0) {
-  int hb;
-  map_cblock(blockIdx.x, gridDim.x, c, &hb, M / B);
-  *cb = hb / (kFftBatch / B);
-  *col0 = (hb % (kFftBatch / B)) * B;
-  *k0 = hb * B;
-}
-
 // As k_col_fwd of asm_fft.hip.  A thread's U butterflies of the innermost
 // stage (radix R) own U R spectrum elements through the plane loop.
 template <int R, int U, int B>

@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "fast_trig.h"
 #include "hrf_internal.h"
 
 namespace hrf {
@@ -73,6 +74,51 @@ __device__ __forceinline__ void map_cblock(int bid, int nblk, int* chan, int* cb
   const int logical = (x < r) ? x * (q + 1) + i : r * (q + 1) + (x - r) * q + i;
   *chan = logical / ncb;
   *cb = logical - (*chan) * ncb;
+}
+
+// kz of spectral element (row frequency i, column frequency k), -1 where the
+// evanescent cut or the aperture zeroes the transfer function.
+__device__ __forceinline__ float kz_or_cut(float k0, int i, int k, int M, float sfreq, float ap) {
+  float fx, fy;
+  bool inap, prop;
+  coords(i, k, M, sfreq, ap, &fx, &fy, &inap);
+  const float kk = kz_of(k0, fx, fy, &prop);
+  return prop && inap ? kk : -1.0f;
+}
+
+struct Band {
+  float fxm, fym, d;
+  bool all;
+};
+__device__ __forceinline__ Band band_of(const AsmFftConsts& mc, int p, int c) {
+  return Band{mc.fxmax[p * kMaxChannels + c], mc.fymax[p * kMaxChannels + c], mc.d[p],
+              mc.band_all[p * kMaxChannels + c] != 0};
+}
+// Whether the transfer function passes (i, k), given its kz.
+__device__ __forceinline__ bool passes(const Band& bd, float kz, int i, int k, int M,
+                                       float sfreq) {
+  if (kz < 0.0f) return false;
+  if (bd.all) return true;
+  float fx, fy;
+  bool inap;
+  coords(i, k, M, sfreq, -1.0f, &fx, &fy, &inap);
+  return fabsf(fx) < bd.fxm && fabsf(fy) < bd.fym;
+}
+__device__ __forceinline__ float2 turn(float2 x, float phase) {
+  float sn, cs;
+  sincos_big_ff(phase, &sn, &cs);
+  return make_float2(x.x * cs - x.y * sn, x.x * sn + x.y * cs);
+}
+
+// The block's channel, intermediate tile, first column in it and first
+// spectrum column.
+template <int B>
+__device__ __forceinline__ void column_block(int M, int* c, int* cb, int* col0, int* k0) {
+  int hb;
+  map_cblock(blockIdx.x, gridDim.x, c, &hb, M / B);
+  *cb = hb / (kFftBatch / B);
+  *col0 = (hb % (kFftBatch / B)) * B;
+  *k0 = hb * B;
 }
 
 inline AsmFftConsts fft_consts(int P, int C, int M, double pitch, const float* wl, const float* dist) {
