@@ -1,0 +1,339 @@
+// asm_col.h — column passes of the planned lengths whose transforms work in
+// place: decimation in frequency forward (natural order in, digit-reversed
+// out), decimation in time inverse, radices R1, R2, RL.
+//
+// Against a Stockham transform (asm_fft.hip) a butterfly writes back to the
+// places it read, so a stage takes one barrier instead of two and holds nothing
+// across it; the innermost forward stage hands its outputs to the transfer
+// function in registers, and the innermost inverse stage takes them from
+// there, so a plane's transform costs four LDS accesses per element instead of
+// seven, and three barriers instead of six.  The spectrum's digit-reversed
+// order never matters: a position's frequency is a few digits.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include "asm_common.h"
+#include "fast_trig.h"
+#include "fft_dft.h"
+#include "hrf_internal.h"
+
+namespace hrf {
+namespace {
+
+// R1, R2, RL: radices (product N); kB: columns per block; kT: threads, one per
+// butterfly of the innermost stage; kPad: elements of LDS padding after every
+// 16 (lengths whose innermost radix is a power of two: its butterflies'
+// accesses would otherwise start on the same banks); kWaves: waves per SIMD
+// that the registers are limited for.
+template <int N>
+struct InPlace {
+  static constexpr bool kFwd = false, kAdj = false;  // which of the two passes work in place
+};
+template <int RR1, int RR2, int RRL, int BB, int PP, int WW>
+struct InPlacePlan {
+  static constexpr int R1 = RR1, R2 = RR2, RL = RRL, kB = BB, kPad = PP, kWaves = WW;
+  static constexpr int kN = R1 * R2 * RL, kD1 = R2 * RL, kD2 = RL;
+  static constexpr int kT = (kB * (kN / RL) + 63) / 64 * 64;
+  // LDS index of element i; a transform's line starts at a multiple of kLd.
+  // An 8-byte access serves 16 lanes at a time from 32 banks, here 16 / kB
+  // consecutive elements of kB lines: kLd modulo 16 elements (128 bytes) puts
+  // the lines side by side.
+  __host__ __device__ static constexpr int at(int i) { return kPad ? i + i / 16 * kPad : i; }
+  static constexpr int kLen = at(kN - 1) + 1;
+  static constexpr int kWant = 16 / kB;
+  static constexpr int kLd = kLen + (kWant - kLen % 16 + 16) % 16;
+  static_assert(!kPad || (kD1 % 16 == 0 && kD2 % 16 == 0) || (kD1 % 16 == 0 && 16 % kD2 == 0),
+                "padding stays linear in a butterfly's index");
+  static constexpr int kTw = (R1 - 1) * kD1 + (R2 - 1) * kD2;  // twiddles of both outer stages
+};
+// Which lengths: microseconds of the forward and adjoint column pass of nine
+// fields, Stockham (8 8 8 8 and 16 16 5 3 in 1024-thread blocks, 8 8 8 4) against
+// in place: 4096 573 / 524 -> 433 / 440, 3840 593 / 545 -> 440 / 424, 2048 119 / 98
+// -> 104 / 104 (only the forward is taken).  At 2016 (16 14 9: 247 / 196 -> 240 /
+// 247) and 1600 (16 10 10: 76 / 73 -> 88 / 97) the Stockham passes stay: these
+// plans' blocks of 7 or 10 waves fill a CU badly at the registers they need
+// (one thread per innermost butterfly: 448, 320 or 640), and without the
+// Stockham passes' sharing of kz and sine and cosine between row mirrors they
+// issue as many instructions.
+#define HRF_INPLACE_PLANS(X)             \
+  X(2048, true, false, 16, 16, 8, 2, 2, 4)   \
+  X(3840, true, true, 16, 16, 15, 2, 0, 4)   \
+  X(4096, true, true, 16, 16, 16, 2, 2, 4)
+#define HRF_INPLACE(NN, FWD, ADJ, ...)                       \
+  template <>                                                \
+  struct InPlace<NN> : InPlacePlan<__VA_ARGS__> {            \
+    static constexpr bool kFwd = FWD, kAdj = ADJ;            \
+  };
+HRF_INPLACE_PLANS(HRF_INPLACE)
+#undef HRF_INPLACE
+
+// A stage starts from an opaque thread index, so that the compiler does not
+// hoist its addresses out of the plane loop and hold them in registers.
+__device__ __forceinline__ unsigned stage_tid() {
+  unsigned tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  return tid;
+}
+
+// Outermost forward stage, inputs from in(position, column).  HALF: the
+// inputs at t < R1 / 4 and t >= 3 R1 / 4 are zero (R1 = 16).
+template <class PL, bool HALF, class In>
+__device__ __forceinline__ void ip_first(float2* lds, const float2* __restrict__ tw, In& in) {
+  constexpr int R = PL::R1, D = PL::kD1, B = PL::kB, NB = B * D, T = PL::kT;
+  constexpr int SP = D + (PL::kPad ? D / 16 * PL::kPad : 0);
+  static_assert(!HALF || R == 16, "pruned first stage");
+  const unsigned tid = stage_tid();
+#pragma unroll
+  for (int u = 0; u < (NB + T - 1) / T; ++u) {
+    const unsigned q = tid + u * T;
+    if (NB % T == 0 || q < static_cast<unsigned>(NB)) {
+      const unsigned j = q / B, b = q % B;
+      float2 x[R];
+#pragma unroll
+      for (int t = 0; t < R; ++t)
+        if (!HALF || (t >= R / 4 && t < 3 * R / 4))
+          x[t] = in(static_cast<int>(j) + t * D, static_cast<int>(b));
+      if constexpr (HALF)
+        dft16<false, true>(x);
+      else
+        Dft<R, false>::run(x);
+      float2* p = lds + (b * PL::kLd + PL::at(static_cast<int>(j)));
+      p[0] = x[0];
+#pragma unroll
+      for (int t = 1; t < R; ++t) p[t * SP] = cmulf(x[t], tw[(t - 1) * D + j]);
+    }
+  }
+}
+
+// Middle stage in place (DIT: conjugate twiddles before the butterfly).
+template <class PL, bool DIT>
+__device__ __forceinline__ void ip_middle(float2* lds, const float2* __restrict__ tw) {
+  constexpr int R = PL::R2, D = PL::kD2, B = PL::kB, NB = B * PL::R1 * D, T = PL::kT;
+  constexpr int SP = D % 16 == 0 ? D + (PL::kPad ? D / 16 * PL::kPad : 0) : D;
+  const float2* w = tw + (PL::R1 - 1) * PL::kD1;
+  const unsigned tid = stage_tid();
+#pragma unroll
+  for (int u = 0; u < (NB + T - 1) / T; ++u) {
+    const unsigned q = tid + u * T;
+    if (NB % T == 0 || q < static_cast<unsigned>(NB)) {
+      const unsigned j = q / B, b = q % B, hi = j / D, lo = j % D;
+      unsigned a = b * PL::kLd + PL::at(static_cast<int>(hi * (D * R) + lo));
+      float2 x[R];
+      // with padding and D < 16 the padding steps inside the butterfly
+      auto off = [](int t) {
+        return (PL::kPad && D % 16 != 0) ? PL::at(t * D) : t * SP;
+      };
+#pragma unroll
+      for (int t = 0; t < R; ++t) x[t] = lds[a + off(t)];
+      if (DIT) {
+#pragma unroll
+        for (int t = 1; t < R; ++t) {
+          const float2 v = w[(t - 1) * D + lo];
+          x[t] = cmulf(x[t], make_float2(v.x, -v.y));
+        }
+      }
+      Dft<R, DIT>::run(x);
+      if (!DIT) {
+#pragma unroll
+        for (int t = 1; t < R; ++t) x[t] = cmulf(x[t], w[(t - 1) * D + lo]);
+      }
+#pragma unroll
+      for (int t = 0; t < R; ++t) lds[a + off(t)] = x[t];
+    }
+  }
+}
+
+// Outermost inverse stage, outputs to out(position, column, value).
+template <class PL, class Out>
+__device__ __forceinline__ void ip_last(const float2* lds, const float2* __restrict__ tw,
+                                        Out& out) {
+  constexpr int R = PL::R1, D = PL::kD1, B = PL::kB, NB = B * D, T = PL::kT;
+  constexpr int SP = D + (PL::kPad ? D / 16 * PL::kPad : 0);
+  const unsigned tid = stage_tid();
+#pragma unroll
+  for (int u = 0; u < (NB + T - 1) / T; ++u) {
+    const unsigned q = tid + u * T;
+    if (NB % T == 0 || q < static_cast<unsigned>(NB)) {
+      const unsigned j = q / B, b = q % B;
+      const float2* p = lds + (b * PL::kLd + PL::at(static_cast<int>(j)));
+      float2 x[R];
+      x[0] = p[0];
+#pragma unroll
+      for (int t = 1; t < R; ++t) {
+        const float2 v = tw[(t - 1) * D + j];
+        x[t] = cmulf(p[t * SP], make_float2(v.x, -v.y));
+      }
+      Dft<R, true>::run(x);
+#pragma unroll
+      for (int t = 0; t < R; ++t) out(static_cast<int>(j) + t * D, static_cast<int>(b), x[t]);
+    }
+  }
+}
+
+// A thread's innermost butterfly: its RL elements in LDS, its column, and the
+// row frequency of its first element (element t: fb + t N / RL).
+template <class PL>
+struct Inner {
+  float2* p;
+  int b, fb;
+  bool on;
+  __device__ __forceinline__ Inner(float2* lds, unsigned tid) {
+    const int j = static_cast<int>(tid / PL::kB);
+    b = static_cast<int>(tid % PL::kB);
+    on = PL::kT == PL::kB * (PL::kN / PL::RL) || j < PL::kN / PL::RL;
+    p = lds + (b * PL::kLd + PL::at(j * PL::RL));
+    fb = j / PL::R2 + j % PL::R2 * PL::R1;
+  }
+  __device__ __forceinline__ void load(float2 (&x)[PL::RL]) const {
+    if constexpr (PL::RL % 2 == 0) {
+#pragma unroll
+      for (int t = 0; t < PL::RL; t += 2) {
+        const float4 v = *reinterpret_cast<const float4*>(p + t);
+        x[t] = make_float2(v.x, v.y);
+        x[t + 1] = make_float2(v.z, v.w);
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < PL::RL; ++t) x[t] = p[t];
+    }
+  }
+  __device__ __forceinline__ void store(const float2 (&x)[PL::RL]) const {
+    if constexpr (PL::RL % 2 == 0) {
+#pragma unroll
+      for (int t = 0; t < PL::RL; t += 2)
+        *reinterpret_cast<float4*>(p + t) = make_float4(x[t].x, x[t].y, x[t + 1].x, x[t + 1].y);
+    } else {
+#pragma unroll
+      for (int t = 0; t < PL::RL; ++t) p[t] = x[t];
+    }
+  }
+};
+
+template <class PL>
+__device__ __forceinline__ void ip_kz(const Inner<PL>& in, float k0, int kcol, float sfreq,
+                                      float ap, float (&kz)[PL::RL]) {
+#pragma unroll
+  for (int t = 0; t < PL::RL; ++t)
+    kz[t] = in.on ? kz_or_cut(k0, in.fb + t * (PL::R1 * PL::R2), kcol, PL::kN, sfreq, ap) : -1.0f;
+}
+
+// The passes B and B' of asm_fft.hip (same arguments and layouts).
+template <int N, bool HALF>
+__global__ __launch_bounds__(InPlace<N>::kT, InPlace<N>::kWaves) void k_col_fwd_ip(
+    const float2* __restrict__ X, float2* __restrict__ Z, int P, int C, int H, int r_pad, int S,
+    int s_crop, float sfreq, float ap, AsmFftConsts mc, const float2* __restrict__ tw,
+    int accumulate) {
+  using PL = InPlace<N>;
+  constexpr int B = PL::kB, RL = PL::RL, K = PL::R1 * PL::R2;
+  __shared__ __align__(16) float2 lds[B * PL::kLd];
+  int c, cb, col0, k0;
+  column_block<B>(N, &c, &cb, &col0, &k0);
+  constexpr int ncb = N / kFftBatch;
+  const float2* src = X + tile_off(c, ncb, cb, H, 0, 0, kFftBatch) + col0;
+  auto in = [&](int pos, int b) -> float2 {
+    const unsigned r = static_cast<unsigned>(pos - r_pad);
+    return r < static_cast<unsigned>(H) ? src[r * kFftBatch + b] : make_float2(0.0f, 0.0f);
+  };
+  ip_first<PL, HALF>(lds, tw, in);
+  Inner<PL> mine(lds, threadIdx.x);
+  float kz[RL];
+  float2 acc[RL];
+  ip_kz<PL>(mine, mc.k[c], k0 + mine.b, sfreq, ap, kz);
+#pragma unroll
+  for (int t = 0; t < RL; ++t) acc[t] = make_float2(0.0f, 0.0f);
+  for (int p = 0; p < P; ++p) {
+    if (p > 0) {
+      __syncthreads();
+      src = X + tile_off(p * C + c, ncb, cb, H, 0, 0, kFftBatch) + col0;
+      ip_first<PL, HALF>(lds, tw, in);
+    }
+    __syncthreads();
+    ip_middle<PL, false>(lds, tw);
+    __syncthreads();
+    const Band bd = band_of(mc, p, c);
+    Inner<PL> at(lds, stage_tid());
+    if (at.on) {
+      float2 x[RL];
+      at.load(x);
+      Dft<RL, false>::run(x);
+#pragma unroll
+      for (int t = 0; t < RL; ++t)
+        if (passes(bd, kz[t], at.fb + t * K, k0 + at.b, N, sfreq))
+          acc[t] = cadd(acc[t], turn(x[t], bd.d * kz[t]));
+    }
+  }
+  __syncthreads();
+  if (mine.on) {
+    Dft<RL, true>::run(acc);
+    mine.store(acc);
+  }
+  __syncthreads();
+  ip_middle<PL, true>(lds, tw);
+  __syncthreads();
+  float2* dst = Z + tile_off(c, ncb, cb, S, 0, 0, kFftBatch) + col0;
+  auto out = [&](int pos, int b, float2 v) {
+    const unsigned r = static_cast<unsigned>(pos - s_crop);
+    if (r < static_cast<unsigned>(S)) {
+      float2* o = dst + r * kFftBatch + b;
+      *o = accumulate ? cadd(*o, v) : v;
+    }
+  };
+  ip_last<PL>(lds, tw, out);
+}
+
+template <int N, bool HALF>
+__global__ __launch_bounds__(InPlace<N>::kT, InPlace<N>::kWaves) void k_col_adj_ip(
+    const float2* __restrict__ X, float2* __restrict__ Z, int P, int C, int S, int s_pad, int H,
+    int r_crop, float sfreq, float ap, AsmFftConsts mc, const float2* __restrict__ tw) {
+  using PL = InPlace<N>;
+  constexpr int B = PL::kB, RL = PL::RL, K = PL::R1 * PL::R2;
+  __shared__ __align__(16) float2 lds[B * PL::kLd];
+  int c, cb, col0, k0;
+  column_block<B>(N, &c, &cb, &col0, &k0);
+  constexpr int ncb = N / kFftBatch;
+  const float2* src = X + tile_off(c, ncb, cb, S, 0, 0, kFftBatch) + col0;
+  auto in = [&](int pos, int b) -> float2 {
+    const unsigned r = static_cast<unsigned>(pos - s_pad);
+    return r < static_cast<unsigned>(S) ? src[r * kFftBatch + b] : make_float2(0.0f, 0.0f);
+  };
+  ip_first<PL, HALF>(lds, tw, in);
+  Inner<PL> mine(lds, threadIdx.x);
+  float kz[RL];
+  float2 g[RL];
+  ip_kz<PL>(mine, mc.k[c], k0 + mine.b, sfreq, ap, kz);
+  __syncthreads();
+  ip_middle<PL, false>(lds, tw);
+  __syncthreads();
+  if (mine.on) {
+    mine.load(g);
+    Dft<RL, false>::run(g);
+  }
+  for (int p = 0; p < P; ++p) {
+    __syncthreads();
+    const Band bd = band_of(mc, p, c);
+    Inner<PL> at(lds, stage_tid());
+    if (at.on) {
+      float2 x[RL];
+#pragma unroll
+      for (int t = 0; t < RL; ++t)
+        x[t] = passes(bd, kz[t], at.fb + t * K, k0 + at.b, N, sfreq)
+                   ? turn(g[t], -bd.d * kz[t])
+                   : make_float2(0.0f, 0.0f);
+      Dft<RL, true>::run(x);
+      at.store(x);
+    }
+    __syncthreads();
+    ip_middle<PL, true>(lds, tw);
+    __syncthreads();
+    float2* dst = Z + tile_off(p * C + c, ncb, cb, H, 0, 0, kFftBatch) + col0;
+    auto out = [&](int pos, int b, float2 v) {
+      const unsigned r = static_cast<unsigned>(pos - r_crop);
+      if (r < static_cast<unsigned>(H)) dst[r * kFftBatch + b] = v;
+    };
+    ip_last<PL>(lds, tw, out);
+  }
+}
+
+}  // namespace
+}  // namespace hrf

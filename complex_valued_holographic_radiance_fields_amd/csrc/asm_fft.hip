@@ -22,8 +22,9 @@
 // batch of B rows or columns held in LDS: each stage reads all butterfly
 // inputs into registers, applies table twiddles (double-precision table,
 // rounded to float), does the R-point DFT, and writes the outputs back to
-// their Stockham positions between two barriers.  Transform lengths
-// without a plan here use the hipFFT path.
+// their Stockham positions between two barriers.  The longest column passes
+// work in place instead (asm_col.h); lengths without a plan here take the
+// passes of asm_any.hip.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -31,6 +32,7 @@
 #include <mutex>
 #include <vector>
 
+#include "asm_col.h"
 #include "asm_common.h"
 #include "fast_trig.h"
 #include "fft_dft.h"
@@ -47,17 +49,10 @@ template <int N>
 constexpr int kRowBatch = N > 1600 ? 2 : 4;
 template <int N>
 constexpr int kRowThreads = 256 * kRowBatch<N>;
-// Column-pass threads and the occupancy they are compiled for: the longest
-// transforms (N >= 3840: a 138-147 KB LDS batch, one block per CU) run
-// twice the waves per block, which also halves each thread's share of the
-// per-element transfer state.
-template <int N>
-constexpr int kColThreads = N >= 3840 ? 1024 : kFftThreads;
 // Columns per column-pass block: two (half an intermediate tile) above
-// 1600 points, where a four-column batch takes 73-147 KB of LDS (one or two
-// blocks per CU) and, at 3840/4096, 16 spectrum and transfer entries per
-// thread (spilled); four at 1600 and below (two columns measured no faster
-// at 1600).
+// 1600 points, where a four-column batch takes 73 KB of LDS or more (two
+// blocks per CU); four at 1600 and below (two columns measured no faster at
+// 1600).
 template <int N>
 constexpr int kColBatch = N > 1600 ? 2 : kFftBatch;
 template <int N>
@@ -428,60 +423,10 @@ struct Plan;
 HRF_FFT_PLANS(HRF_FFT_PLAN)
 #undef HRF_FFT_PLAN
 
-// Plans of the column passes where they differ from the length's: at 4096
-// points the column blocks (1024 threads, two transforms) would leave half
-// their waves idle in every radix-16 stage (512 butterflies), so they keep
-// 8 8 8 8, while the row passes (512 threads) take 16 16 16.
-#define HRF_FFT_COL_PLANS(X) X(4096, 8, 8, 8, 8)
-template <int N>
-struct PlanCol : Plan<N> {};
-#define HRF_FFT_PLAN(NN, ...)                                                       \
-  template <>                                                                       \
-  struct PlanCol<NN> {                                                              \
-    template <int B>                                                                \
-    static constexpr int kPad = kPadSlots<first_radix(__VA_ARGS__), B>;             \
-    template <bool INV, int T = kFftThreads, bool HALF = false, int B = kFftBatch>  \
-    __device__ __forceinline__ static void run(float2* lds, const float2* tw) {     \
-      run_stages<T, B, kPad<B>, NN, INV, HALF, 1, 0, __VA_ARGS__>(lds, tw);         \
-    }                                                                               \
-    template <bool INV, int T, bool HALF, int B, class In>                          \
-    __device__ __forceinline__ static void run_in(float2* lds, const float2* tw,    \
-                                                  In& in) {                         \
-      run_stages_in<T, B, kPad<B>, NN, INV, HALF, In, __VA_ARGS__>(lds, tw, in);    \
-    }                                                                               \
-    static constexpr int kR1 = first_radix(__VA_ARGS__);                            \
-    template <int T, bool HALF, int B, class In>                                    \
-    __device__ __forceinline__ static void load_first(In& in, float2 (&x)[kR1]) {   \
-      first_stage_load<NN, kR1, T, HALF, B>(in, x);                                 \
-    }                                                                               \
-    template <bool INV, int T, bool HALF, int B>                                    \
-    __device__ __forceinline__ static void run_from(float2* lds, const float2* tw,  \
-                                                    float2 (&x)[kR1]) {             \
-      run_stages_from<T, B, kPad<B>, NN, INV, HALF, __VA_ARGS__>(lds, tw, x);       \
-    }                                                                               \
-    template <bool INV, int T, bool HALF, int B, class In, class Out>               \
-    __device__ __forceinline__ static void run_in_out(float2* lds, const float2* tw,\
-                                                      In& in, Out& out) {           \
-      run_stages_in_out<T, B, kPad<B>, NN, INV, HALF, In, Out, __VA_ARGS__>(lds, tw,\
-                                                                 in, out);          \
-    }                                                                               \
-    template <bool INV, int T, int B, class Out>                                    \
-    __device__ __forceinline__ static void run_out(float2* lds, const float2* tw,   \
-                                                   Out& out) {                      \
-      run_stages_out<T, B, kPad<B>, NN, INV, 1, 0, Out, __VA_ARGS__>(lds, tw, out); \
-    }                                                                               \
-  };
-HRF_FFT_COL_PLANS(HRF_FFT_PLAN)
-#undef HRF_FFT_PLAN
-
-// Host: the radix sequence of a plan (empty for lengths without one); col:
-// the column passes' plan.
-std::vector<int> plan_radices(int N, bool col) {
+// Host: the radix sequence of a plan (empty for lengths without one).
+std::vector<int> plan_radices(int N) {
 #define HRF_FFT_RADICES(NN, ...) \
   if (N == NN) return std::vector<int>{__VA_ARGS__};
-  if (col) {
-    HRF_FFT_COL_PLANS(HRF_FFT_RADICES)
-  }
   HRF_FFT_PLANS(HRF_FFT_RADICES)
 #undef HRF_FFT_RADICES
   return {};
@@ -590,15 +535,15 @@ __global__ __launch_bounds__(kRowThreads<N>) void k_rows_out(const float2* __res
 // HALF: the field rows lie in [N/4, 3N/4); only that half is staged and the
 // forward transforms' first stage is pruned.
 template <int N, bool HALF>
-__global__ __launch_bounds__(kColThreads<N>, kColMinBlocks<N>) void k_col_fwd(
+__global__ __launch_bounds__(kFftThreads, kColMinBlocks<N>) void k_col_fwd(
     const float2* __restrict__ X, float2* __restrict__ Z, int P, int C, int H, int r_pad, int S,
     int s_crop, float sfreq, float ap, AsmFftConsts mc, const float2* __restrict__ tw,
     int accumulate) {
   constexpr int B = kColBatch<N>;  // columns of this block
   constexpr int TB = kFftBatch;    // columns of an intermediate tile
-  constexpr int T = kColThreads<N>;
+  constexpr int T = kFftThreads;
   constexpr int ncb = N / TB;
-  __shared__ float2 lds[lds_elems<N, B, PlanCol<N>::template kPad<B>>()];
+  __shared__ float2 lds[lds_elems<N, B, Plan<N>::template kPad<B>>()];
   __shared__ float2 s_tw[kTwLdsElems<N>];
   const float2* twp = stage_twiddles<N, T>(s_tw, tw);
   int c, hb;
@@ -616,15 +561,15 @@ __global__ __launch_bounds__(kColThreads<N>, kColMinBlocks<N>) void k_col_fwd(
   // aperture zeroes the transfer function of both elements for every plane.
   // kSplit: the first plane's first-stage loads are issued before the kz
   // prologue, so its arithmetic overlaps their latency (half-grid inputs at
-  // the lengths where the registers the loads hold cost no occupancy).
-  constexpr bool kSplit = HALF && (N == 1600 || N == 3840 || N == 4096);
+  // 1600 points, where the registers the loads hold cost no occupancy).
+  constexpr bool kSplit = HALF && N == 1600;
   const float2* src = X + tile_off(c, ncb, cb, H, 0, 0, TB) + col0;
   auto in = [&](int pos, int b) -> float2 {
     const unsigned r = static_cast<unsigned>(pos - r_pad);
     return r < static_cast<unsigned>(H) ? src[r * TB + b] : make_float2(0.0f, 0.0f);
   };
-  float2 xin[PlanCol<N>::kR1];
-  if constexpr (kSplit) PlanCol<N>::template load_first<T, HALF, B>(in, xin);
+  float2 xin[Plan<N>::kR1];
+  if constexpr (kSplit) Plan<N>::template load_first<T, HALF, B>(in, xin);
   constexpr int NS = (N / 2 + 1) * B;  // slots
   constexpr int SPT = (NS + T - 1) / T;
   static_assert(2 * SPT <= 32, "two aperture bits per slot in one word");
@@ -659,9 +604,9 @@ __global__ __launch_bounds__(kColThreads<N>, kColMinBlocks<N>) void k_col_fwd(
     __syncthreads();
     src = X + tile_off(p * C + c, ncb, cb, H, 0, 0, TB) + col0;
     if (kSplit && p == 0)
-      PlanCol<N>::template run_from<false, T, HALF, B>(lds, twp, xin);
+      Plan<N>::template run_from<false, T, HALF, B>(lds, twp, xin);
     else
-      PlanCol<N>::template run_in<false, T, HALF, B>(lds, twp, in);
+      Plan<N>::template run_in<false, T, HALF, B>(lds, twp, in);
     const float fxm = mc.fxmax[p * kMaxChannels + c], fym = mc.fymax[p * kMaxChannels + c];
     const bool band_all = mc.band_all[p * kMaxChannels + c] != 0;
     const float d = mc.d[p];
@@ -688,13 +633,13 @@ __global__ __launch_bounds__(kColThreads<N>, kColMinBlocks<N>) void k_col_fwd(
           float sn, cs;
           sincos_big_ff(d * kz[u], &sn, &cs);
           if ((amask >> (2 * u)) & 1u) {
-            const float2 x = lds[pad<PlanCol<N>::template kPad<B>>(q)];
+            const float2 x = lds[pad<Plan<N>::template kPad<B>>(q)];
             acc[u].x += x.x * cs - x.y * sn;
             acc[u].y += x.x * sn + x.y * cs;
           }
           if ((amask >> (2 * u + 1)) & 1u) {
             const float2 x2 =
-                lds[pad<PlanCol<N>::template kPad<B>>((N - q / B) * B + q % B)];
+                lds[pad<Plan<N>::template kPad<B>>((N - q / B) * B + q % B)];
             acc2[u].x += x2.x * cs - x2.y * sn;
             acc2[u].y += x2.x * sn + x2.y * cs;
           }
@@ -707,9 +652,9 @@ __global__ __launch_bounds__(kColThreads<N>, kColMinBlocks<N>) void k_col_fwd(
   for (int u = 0; u < SPT; ++u) {
     const int q = threadIdx.x + u * T;
     if (q < NS) {
-      lds[pad<PlanCol<N>::template kPad<B>>(q)] = acc[u];
+      lds[pad<Plan<N>::template kPad<B>>(q)] = acc[u];
       const int i = q / B;
-      if (i != 0 && i != N / 2) lds[pad<PlanCol<N>::template kPad<B>>((N - i) * B + q % B)] = acc2[u];
+      if (i != 0 && i != N / 2) lds[pad<Plan<N>::template kPad<B>>((N - i) * B + q % B)] = acc2[u];
     }
   }
   __syncthreads();
@@ -723,7 +668,7 @@ __global__ __launch_bounds__(kColThreads<N>, kColMinBlocks<N>) void k_col_fwd(
       *o = accumulate ? cadd(*o, v) : v;
     }
   };
-  PlanCol<N>::template run_out<true, T, B>(lds, twp, out);
+  Plan<N>::template run_out<true, T, B>(lds, twp, out);
 }
 
 // B': adjoint column pass.  X tiled (C, S, N) row spectra of the padded
@@ -732,14 +677,14 @@ __global__ __launch_bounds__(kColThreads<N>, kColMinBlocks<N>) void k_col_fwd(
 // HALF: the S gradient rows lie in [N/4, 3N/4) (always, with N = 2S); only
 // that half is staged and the forward transform's first stage is pruned.
 template <int N, bool HALF>
-__global__ __launch_bounds__(kColThreads<N>, kColMinBlocks<N>) void k_col_adj(
+__global__ __launch_bounds__(kFftThreads, kColMinBlocks<N>) void k_col_adj(
     const float2* __restrict__ X, float2* __restrict__ Z, int P, int C, int S, int s_pad, int H,
     int r_crop, float sfreq, float ap, AsmFftConsts mc, const float2* __restrict__ tw) {
   constexpr int B = kColBatch<N>;
   constexpr int TB = kFftBatch;
-  constexpr int T = kColThreads<N>;
+  constexpr int T = kFftThreads;
   constexpr int ncb = N / TB;
-  __shared__ float2 lds[lds_elems<N, B, PlanCol<N>::template kPad<B>>()];
+  __shared__ float2 lds[lds_elems<N, B, Plan<N>::template kPad<B>>()];
   __shared__ float2 s_tw[kTwLdsElems<N>];
   const float2* twp = stage_twiddles<N, T>(s_tw, tw);
   int c, hb;
@@ -755,14 +700,14 @@ __global__ __launch_bounds__(kColThreads<N>, kColMinBlocks<N>) void k_col_adj(
     return r < static_cast<unsigned>(S) ? src[r * TB + b] : make_float2(0.0f, 0.0f);
   };
   // kSplit: the first stage's loads are issued before the kz prologue, so
-  // its arithmetic overlaps their latency (half-grid inputs at the lengths
+  // its arithmetic overlaps their latency (half-grid inputs at 1600 points,
   // where the registers the loads hold cost no occupancy).
-  constexpr bool kSplit = HALF && (N == 1600 || N == 3840 || N == 4096);
-  float2 xin[PlanCol<N>::kR1];
+  constexpr bool kSplit = HALF && N == 1600;
+  float2 xin[Plan<N>::kR1];
   if constexpr (kSplit)
-    PlanCol<N>::template load_first<T, HALF, B>(in, xin);
+    Plan<N>::template load_first<T, HALF, B>(in, xin);
   else
-    PlanCol<N>::template run_in<false, T, HALF, B>(lds, twp, in);
+    Plan<N>::template run_in<false, T, HALF, B>(lds, twp, in);
   // Slots own an element and its row mirror, as in k_col_fwd.
   constexpr int NS = (N / 2 + 1) * B;
   constexpr int SPT = (NS + T - 1) / T;
@@ -788,7 +733,7 @@ __global__ __launch_bounds__(kColThreads<N>, kColMinBlocks<N>) void k_col_adj(
       amask |= (in1 ? 1u : 0u) << (2 * u) | (in2 ? 1u : 0u) << (2 * u + 1);
     }
   }
-  if constexpr (kSplit) PlanCol<N>::template run_from<false, T, HALF, B>(lds, twp, xin);
+  if constexpr (kSplit) Plan<N>::template run_from<false, T, HALF, B>(lds, twp, xin);
 #pragma unroll
   for (int u = 0; u < SPT; ++u) {
     const int q = threadIdx.x + u * T;
@@ -796,8 +741,8 @@ __global__ __launch_bounds__(kColThreads<N>, kColMinBlocks<N>) void k_col_adj(
     gs2[u] = make_float2(0.0f, 0.0f);
     if (q < NS) {
       const int i = q / B, b = q % B;
-      gs[u] = lds[pad<PlanCol<N>::template kPad<B>>(q)];
-      if (i != 0 && i != N / 2) gs2[u] = lds[pad<PlanCol<N>::template kPad<B>>((N - i) * B + b)];
+      gs[u] = lds[pad<Plan<N>::template kPad<B>>(q)];
+      if (i != 0 && i != N / 2) gs2[u] = lds[pad<Plan<N>::template kPad<B>>((N - i) * B + b)];
     }
   }
   for (int p = 0; p < P; ++p) {
@@ -828,9 +773,9 @@ __global__ __launch_bounds__(kColThreads<N>, kColMinBlocks<N>) void k_col_adj(
               r2 = make_float2(gs2[u].x * cs - gs2[u].y * sn, gs2[u].x * sn + gs2[u].y * cs);
           }
         }
-        lds[pad<PlanCol<N>::template kPad<B>>(q)] = r;
+        lds[pad<Plan<N>::template kPad<B>>(q)] = r;
         const int i = q / B;
-        if (i != 0 && i != N / 2) lds[pad<PlanCol<N>::template kPad<B>>((N - i) * B + q % B)] = r2;
+        if (i != 0 && i != N / 2) lds[pad<Plan<N>::template kPad<B>>((N - i) * B + q % B)] = r2;
       }
     }
     __syncthreads();
@@ -841,7 +786,7 @@ __global__ __launch_bounds__(kColThreads<N>, kColMinBlocks<N>) void k_col_adj(
       const unsigned r = static_cast<unsigned>(pos - r_crop);
       if (r < static_cast<unsigned>(H)) dst[r * TB + b] = v;
     };
-    PlanCol<N>::template run_out<true, T, B>(lds, twp, out);
+    Plan<N>::template run_out<true, T, B>(lds, twp, out);
   }
 }
 
@@ -852,13 +797,12 @@ std::map<std::pair<int, int>, float2*>& tw_tables() {
   return m;
 }
 
-// The twiddle table of the length-N plan (col: the column passes' plan),
-// built once per device.
-int twiddles(int N, const float2** out, bool col = false) {
+// The twiddle table of the length-N plan, built once per device.
+int twiddles(int N, const float2** out) {
   int dev = 0;
   HRF_HIP(hipGetDevice(&dev));
   std::lock_guard<std::mutex> lock(g_tw_mu);
-  auto key = std::make_pair(dev, 2 * N + (col ? 1 : 0));
+  auto key = std::make_pair(dev, 2 * N);
   auto it = tw_tables().find(key);
   if (it != tw_tables().end()) {
     *out = it->second;
@@ -869,7 +813,7 @@ int twiddles(int N, const float2** out, bool col = false) {
   std::vector<float2> h;
   h.reserve(N);
   int ns = 1;
-  for (int r : plan_radices(N, col)) {
+  for (int r : plan_radices(N)) {
     for (int k = 0; k < ns; ++k)
       for (int t = 1; t < r; ++t) {
         const long long m = static_cast<long long>(t) * k * (N / (ns * r));
@@ -889,6 +833,36 @@ int twiddles(int N, const float2** out, bool col = false) {
   HRF_HIP(hipMemcpy(d, h.data(), N * sizeof(float2), hipMemcpyHostToDevice));
   tw_tables()[key] = d;
   *out = d;
+  return HRF_OK;
+}
+
+// Twiddles of an in-place column plan: w(t, lo) = exp(-2 pi i t lo / (D R)) of
+// the outer two stages, at (t - 1) D + lo (asm_col.h), built once per device.
+template <int N>
+int inplace_twiddles(const float2** out) {
+  using PL = InPlace<N>;
+  int dev = 0;
+  HRF_HIP(hipGetDevice(&dev));
+  std::lock_guard<std::mutex> lock(g_tw_mu);
+  auto key = std::make_pair(dev, 2 * N + 1);
+  auto it = tw_tables().find(key);
+  if (it == tw_tables().end()) {
+    std::vector<float2> h;
+    h.reserve(PL::kTw);
+    const int radix[2] = {PL::R1, PL::R2}, span[2] = {PL::kD1, PL::kD2};
+    for (int s = 0; s < 2; ++s)
+      for (int t = 1; t < radix[s]; ++t)
+        for (int lo = 0; lo < span[s]; ++lo) {
+          const double a = -kTwoPiD * static_cast<double>(t * lo) / (radix[s] * span[s]);
+          h.push_back(make_float2(static_cast<float>(std::cos(a)),
+                                  static_cast<float>(std::sin(a))));
+        }
+    float2* d = nullptr;
+    HRF_HIP(hipMalloc(&d, h.size() * sizeof(float2)));
+    HRF_HIP(hipMemcpy(d, h.data(), h.size() * sizeof(float2), hipMemcpyHostToDevice));
+    it = tw_tables().emplace(key, d).first;
+  }
+  *out = it->second;
   return HRF_OK;
 }
 
@@ -927,18 +901,32 @@ template <int N>
 int pass_col_fwd(const float2* X, float2* Z, int P, int C, int h_in, int h_out, float sfreq,
                  float ap, const AsmFftConsts& mc, bool accumulate, hipStream_t s) {
   const float2* tw = nullptr;
-  HRF_TRY(twiddles(N, &tw, true));
-  const dim3 grid(C * (N / kColBatch<N>)), block(kColThreads<N>);
-  if (2 * h_in <= N)
-    hipLaunchKernelGGL((k_col_fwd<N, true>), grid, block, 0, s, X, Z, P, C, h_in,
-                       N / 2 - h_in / 2, h_out, N / 2 - h_out / 2, sfreq, ap, mc, tw,
-                       accumulate ? 1 : 0);
-  else
-    hipLaunchKernelGGL((k_col_fwd<N, false>), grid, block, 0, s, X, Z, P, C, h_in,
-                       N / 2 - h_in / 2, h_out, N / 2 - h_out / 2, sfreq, ap, mc, tw,
-                       accumulate ? 1 : 0);
-  HRF_LAUNCH_CHECK();
-  return HRF_OK;
+  if constexpr (InPlace<N>::kFwd) {
+    using PL = InPlace<N>;
+    HRF_TRY(inplace_twiddles<N>(&tw));
+    const dim3 ipg(C * (N / PL::kB));
+    if (2 * h_in <= N)
+      hipLaunchKernelGGL((k_col_fwd_ip<N, true>), ipg, dim3(PL::kT), 0, s, X, Z, P, C, h_in,
+                         N / 2 - h_in / 2, h_out, N / 2 - h_out / 2, sfreq, ap, mc, tw, accumulate ? 1 : 0);
+    else
+      hipLaunchKernelGGL((k_col_fwd_ip<N, false>), ipg, dim3(PL::kT), 0, s, X, Z, P, C, h_in,
+                         N / 2 - h_in / 2, h_out, N / 2 - h_out / 2, sfreq, ap, mc, tw, accumulate ? 1 : 0);
+    HRF_LAUNCH_CHECK();
+    return HRF_OK;
+  } else {
+    HRF_TRY(twiddles(N, &tw));
+    const dim3 grid(C * (N / kColBatch<N>)), block(kFftThreads);
+    if (2 * h_in <= N)
+      hipLaunchKernelGGL((k_col_fwd<N, true>), grid, block, 0, s, X, Z, P, C, h_in,
+                         N / 2 - h_in / 2, h_out, N / 2 - h_out / 2, sfreq, ap, mc, tw,
+                         accumulate ? 1 : 0);
+    else
+      hipLaunchKernelGGL((k_col_fwd<N, false>), grid, block, 0, s, X, Z, P, C, h_in,
+                         N / 2 - h_in / 2, h_out, N / 2 - h_out / 2, sfreq, ap, mc, tw,
+                         accumulate ? 1 : 0);
+    HRF_LAUNCH_CHECK();
+    return HRF_OK;
+  }
 }
 
 // B' with P transfer functions applied one by one: X (C, h_in, N) ->
@@ -947,16 +935,30 @@ template <int N>
 int pass_col_adj(const float2* X, float2* Z, int P, int C, int h_in, int h_out, float sfreq,
                  float ap, const AsmFftConsts& mc, hipStream_t s) {
   const float2* tw = nullptr;
-  HRF_TRY(twiddles(N, &tw, true));
-  const dim3 grid(C * (N / kColBatch<N>)), block(kColThreads<N>);
-  if (2 * h_in <= N)
-    hipLaunchKernelGGL((k_col_adj<N, true>), grid, block, 0, s, X, Z, P, C, h_in,
-                       N / 2 - h_in / 2, h_out, N / 2 - h_out / 2, sfreq, ap, mc, tw);
-  else
-    hipLaunchKernelGGL((k_col_adj<N, false>), grid, block, 0, s, X, Z, P, C, h_in,
-                       N / 2 - h_in / 2, h_out, N / 2 - h_out / 2, sfreq, ap, mc, tw);
-  HRF_LAUNCH_CHECK();
-  return HRF_OK;
+  if constexpr (InPlace<N>::kAdj) {
+    using PL = InPlace<N>;
+    HRF_TRY(inplace_twiddles<N>(&tw));
+    const dim3 ipg(C * (N / PL::kB));
+    if (2 * h_in <= N)
+      hipLaunchKernelGGL((k_col_adj_ip<N, true>), ipg, dim3(PL::kT), 0, s, X, Z, P, C, h_in,
+                         N / 2 - h_in / 2, h_out, N / 2 - h_out / 2, sfreq, ap, mc, tw);
+    else
+      hipLaunchKernelGGL((k_col_adj_ip<N, false>), ipg, dim3(PL::kT), 0, s, X, Z, P, C, h_in,
+                         N / 2 - h_in / 2, h_out, N / 2 - h_out / 2, sfreq, ap, mc, tw);
+    HRF_LAUNCH_CHECK();
+    return HRF_OK;
+  } else {
+    HRF_TRY(twiddles(N, &tw));
+    const dim3 grid(C * (N / kColBatch<N>)), block(kFftThreads);
+    if (2 * h_in <= N)
+      hipLaunchKernelGGL((k_col_adj<N, true>), grid, block, 0, s, X, Z, P, C, h_in,
+                         N / 2 - h_in / 2, h_out, N / 2 - h_out / 2, sfreq, ap, mc, tw);
+    else
+      hipLaunchKernelGGL((k_col_adj<N, false>), grid, block, 0, s, X, Z, P, C, h_in,
+                         N / 2 - h_in / 2, h_out, N / 2 - h_out / 2, sfreq, ap, mc, tw);
+    HRF_LAUNCH_CHECK();
+    return HRF_OK;
+  }
 }
 
 template <int N>

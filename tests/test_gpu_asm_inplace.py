@@ -1,0 +1,53 @@
+"""Column passes that transform in place (asm_col.h): inputs beyond half the
+grid, where the first stage is not pruned, and the sum into an earlier pass's
+result."""
+import numpy as np
+import pytest
+
+from conftest import rel_l2
+
+pytestmark = pytest.mark.gpu
+
+PITCH = 3.74e-6
+TOL = 2e-6  # float32 transforms of 4096 points both ways: about 3e-7
+
+
+def _z(rng, *s):
+    return (rng.normal(size=s) + 1j * rng.normal(size=s)).astype(np.complex64)
+
+
+@pytest.mark.parametrize("P,H,W,S", [(3, 1500, 10, 1024), (2, 20, 24, 1024), (2, 2200, 6, 1920),
+                                     (1, 2400, 8, 2048), (2, 16, 18, 2048)],
+                         ids=["m2048_tall", "m2048", "m3840_tall", "m4096_tall", "m4096"])
+def test_inplace_columns(hrf, oracle_mod, P, H, W, S):
+    import torch
+    from complex_valued_holographic_radiance_fields_amd import propagation
+
+    print(f"in-place columns M={2 * S} {H}x{W}", flush=True)
+    rng = np.random.default_rng(S + H)
+    wl, dist = [515e-9], [2e-3, -7e-3, 0.0][:P]
+    f, g = _z(rng, P, 1, H, W), _z(rng, 1, S, S)
+    got = propagation.multiplane(torch.from_numpy(f).cuda(), wl, PITCH, dist, (S, S), float(S))
+    ref = oracle_mod.multiplane_forward(f, wl, dist, PITCH, S, float(S))
+    assert rel_l2(got.cpu().numpy(), ref) < TOL
+    adj = propagation.multiplane_adjoint(torch.from_numpy(g).cuda(), (H, W), wl, PITCH, dist,
+                                         (S, S), float(S))
+    assert rel_l2(adj.cpu().numpy(),
+                  oracle_mod.multiplane_adjoint(g, H, W, wl, dist, PITCH, S, float(S))) < TOL
+
+
+@pytest.mark.parametrize("S", [1024, 1920, 2048])
+def test_inplace_accumulates(hrf, monkeypatch, S):
+    import torch
+    from complex_valued_holographic_radiance_fields_amd import _lib, propagation
+
+    rng = np.random.default_rng(S)
+    wl, dist, H, W = [515e-9], [1e-3, -2e-3, 4e-3], 16, 20
+    g = torch.from_numpy(_z(rng, 3, 1, S, S)).cuda()
+    monkeypatch.setattr(propagation, "_MD_EXTRA_BYTES", 0)  # two distances, then one
+    _lib.release_workspaces()
+    adj = propagation.multidistance_adjoint(g, (H, W), wl, PITCH, dist, (S, S), float(S))
+    _lib.release_workspaces()
+    total = sum(propagation.propagate_adjoint(g[d, 0], (H, W), wl[0], PITCH, dv, (S, S), float(S))
+                .cpu().numpy().astype(np.complex128) for d, dv in enumerate(dist))
+    assert rel_l2(adj[0].cpu().numpy(), total) < 1e-6
