@@ -1,0 +1,80 @@
+"""The forward's per-quadrant member lists: each wave of a (tile, plane) block
+composites only the members visible in its own 8x8 pixels.
+
+The scenes put point-like Gaussians (2-D standard deviation 0.55 to 0.65 px, so
+alpha falls below 2^-26 within 4 px) at the centres of chosen quadrants, with
+per-quadrant counts at the edges of the list's padding (groups of 8) and of the
+staged batch (256 list entries), next to wide Gaussians that reach every
+quadrant.  Fields and T against the CPU oracle within 1e-4 relative L2 (the
+rasterizer's fp32 bar: some 100 members, each alpha within 1e-6); where no
+pixel terminates, n_contrib has to equal the oracle's at every pixel, since a
+member that a quadrant skips still counts there."""
+import numpy as np
+import pytest
+
+from conftest import oracle_inputs, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+W, H = 44, 27  # the last tile column and row are partial
+
+
+def _scene(counts, wide, opacity, P, C, seed):
+    """counts: point-like members per quadrant of tile (1, 0); `wide` Gaussians
+    over the whole frame, all shuffled into one depth order."""
+    from complex_valued_holographic_radiance_fields_amd import scenes
+
+    n = sum(counts) + wide
+    sc = scenes.generate(scenes.small("quads", n, W, H, P, C, "uniform", seed=seed))
+    rng = np.random.default_rng(seed)
+    quad = np.repeat(np.arange(5), list(counts) + [wide])
+    rng.shuffle(quad)
+    small = quad < 4
+    u = np.where(small, 16 + 8 * (quad & 1) + 3.5, rng.uniform(0, W, n))
+    v = np.where(small, 8 * ((quad >> 1) & 1) + 3.5, rng.uniform(0, H, n))
+    z = np.sort(rng.uniform(5.0, 9.0, n)).astype(np.float32)
+    m = np.stack([-(u - sc.px) / sc.fx * z, -(v - sc.py) / sc.fy * z, z], 1)
+    sc.cam_means = np.ascontiguousarray(m, np.float32)
+    sc.z = z
+    sig = np.where(small, 0.2, 6.0)[:, None] * np.ones((1, 3))  # pixels
+    sc.scales = np.ascontiguousarray(sig * (z / sc.fx)[:, None], np.float32)
+    sc.opac = np.ascontiguousarray(
+        np.where(rng.random(n) < 0.5, opacity, 0.5 * opacity).reshape(sc.opac.shape), np.float32)
+    return sc
+
+
+COUNTS = [(0, 0, 0, 0), (1, 0, 7, 0), (7, 8, 9, 0), (16, 0, 15, 17), (255, 0, 0, 1),
+          (0, 256, 0, 0), (40, 130, 60, 27), (0, 0, 300, 212)]
+
+
+@pytest.mark.parametrize("P,C", [(1, 1), (2, 2), (3, 3)])
+@pytest.mark.parametrize("opacity", [0.004, 0.9], ids=["live", "terminating"])
+def test_forward_quadrant_lists(hrf, oracle_mod, opacity, P, C):
+    import torch
+    from complex_valued_holographic_radiance_fields_amd import rasterizer, scenes
+
+    for i, counts in enumerate(COUNTS):
+        for wide in (1, 64):
+            sc = _scene(counts, wide, opacity, P, C, seed=5 + i)
+            print(f"P={P} C={C} opacity={opacity} counts={counts} wide={wide}", flush=True)
+            g, cam = oracle_inputs(sc)
+            ref = oracle_mod.rasterize_forward(g, cam)
+            t = scenes.to_torch(sc)
+            field, (fT, nc, pl, ranges, _) = rasterizer.forward(
+                t["cam_means"], t["z"], t["quats"], t["scales"], t["colours"], t["phase"],
+                t["opac"], t["pprobs"], sc.fx, sc.fy, sc.px, sc.py, t["view"], (W, H), (16, 16),
+                1.0, 1000.0)
+            torch.cuda.synchronize()
+            np.testing.assert_array_equal(pl.cpu().numpy(), ref["point_list"])
+            np.testing.assert_array_equal(ranges.cpu().numpy(), ref["ranges"])
+            assert rel_l2(field.cpu().numpy(), ref["field"]) < 1e-4
+            T, Tr = fT.cpu().numpy(), ref["final_T"]
+            assert rel_l2(T, Tr) < 1e-4
+            both = (T < 1e-4) == (Tr < 1e-4)
+            assert np.mean(~both) < 1e-3
+            diff = nc.cpu().numpy() != ref["n_contrib"]
+            if opacity < 0.01:
+                assert not (Tr < 1e-4).any()
+                assert not diff.any()
+            else:
+                assert np.mean(diff) < 1e-3
