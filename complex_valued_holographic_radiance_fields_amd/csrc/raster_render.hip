@@ -396,11 +396,11 @@ __device__ __forceinline__ void render_fwd_block(const RenderParams& p) {
       // The others' alpha stays below 2^-26 at its pixels, so they change
       // neither T nor the end test there.  The member loop is bound by its
       // exponent and blend instructions, and with a projected deviation of
-      // 1-2 px a quadrant sees half of what its tile does: walking the list
-      // instead of the batch takes the kernel from 34.6 to 27.1 us (256^2,
-      // 20,000 Gaussians), 108 to 87 (512^2, 6 planes) and 601 to 512 (1024^2,
-      // 6 planes, 200,000); where Gaussians are wide (800^2, 200,000) the
-      // lists cost nothing (169 to 164).
+      // 1-2 px a quadrant sees about half of what its tile does: walking the
+      // list instead of the batch takes the kernel from 34.6 to 27.1 us
+      // (256^2, 10,000 Gaussians), 108 to 87 (504x378, 250,000, 6 planes) and
+      // 601 to 512 (1008x756, 1 M, 6 planes).  Where Gaussians are wide the
+      // lists cost nothing (800^2, 1 M, 3 planes: 169 to 164).
       const int lane = threadIdx.x & 63;
       const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
       unsigned short* list = s_list[wave];
