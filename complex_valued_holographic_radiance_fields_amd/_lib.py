@@ -100,6 +100,10 @@ SIGNATURES = {
                                         _vp, _vp]),
     "hrf_recon_intensity": (ctypes.c_int, [_vp, _i64, _vp, _vp]),
     "hrf_recon_intensity_backward": (ctypes.c_int, [_vp, _vp, _i64, _vp, _vp]),
+    "hrf_recon_intensity_planes": (ctypes.c_int, [_vp, _i32, _i32, _i32, _i64, _vp, _vp, _vp,
+                                                  _vp, _i32, _vp, _vp]),
+    "hrf_recon_intensity_planes_backward": (ctypes.c_int, [_vp, _vp, _vp, _i32, _i32, _i32, _i64,
+                                                           _vp, _vp, _vp, _vp, _i32, _vp, _vp]),
     "hrf_recon_fields_backward": (ctypes.c_int, [_vp, _vp, _i32, _i32, _i64, _vp, _vp, _vp, _vp,
                                                  _i32, _vp, _vp, _vp, _vp]),
     "hrf_grad_norm_workspace_size": (_sz, [_P(_i64), _i32]),

@@ -14,7 +14,8 @@ The pipeline is four HIP steps: the hologram fields w a e^{i s phi} of the
 band-limited ASM to every depth (each field transformed once for all
 depths, through the multi-plane propagation kernels run with negated
 distances: the fused LDS-FFT passes where the grid size has a plan), the
-intensity (``hrf_recon_intensity``), and the mirror-image backward.  The transfer function is the reference's own band-limited ASM
+intensity straight into the result (``hrf_recon_intensity_planes``), and the
+mirror-image backward.  The transfer function is the reference's own band-limited ASM
 kernel (cuda_prop, the one the rasterizer's hologram uses); the reference's
 reconstruction takes it from odak's ``get_propagation_kernel``, which is not
 available here, so agreement with odak's kernel is not checked.
@@ -49,6 +50,11 @@ def _fan_in(grads, wavelengths, pitch, distances, S, aperture):
                                   aperture)
 
 
+def _batches(parts, dim):
+    """The pair batches' results as one tensor (no copy of a single one)."""
+    return parts[0] if len(parts) == 1 else torch.cat(parts, dim=dim)
+
+
 def _pairs(laser_powers: torch.Tensor, F: int, C: int):
     lp = laser_powers.detach().to("cpu", torch.float32).reshape(F, C)
     pairs = [(f, c, float(lp[f, c])) for f in range(F) for c in range(C) if float(lp[f, c]) != 0]
@@ -73,12 +79,11 @@ class _Reconstruct(torch.autograd.Function):
         D = len(distances)
         hw = S * S
         dev = phases.device
-        out_dtype = torch.complex64 if get_complex else torch.float32
-        out = torch.zeros((F, D, C, S, S), dtype=out_dtype, device=dev)
         ctx.meta = (pairs, scales, wavelengths, pitch, distances, aperture, get_complex, F, C)
         if not pairs:
             ctx.save_for_backward(phases, amplitude, None)
-            return out
+            return torch.zeros((F, D, C, S, S), device=dev,
+                               dtype=torch.complex64 if get_complex else torch.float32)
         K = len(pairs)
         fr, ch, pw, sc = _arrays(pairs, scales)
         lib = _lib.load()
@@ -88,18 +93,19 @@ class _Reconstruct(torch.autograd.Function):
             _lib.check(lib.hrf_recon_fields(amplitude.data_ptr(), phases.data_ptr(), F, C, hw,
                                             fr, ch, pw, sc, K, fields.data_ptr(), stream))
         wl = [wavelengths[c] for _, c, _ in pairs]
-        u = torch.cat([_fan_out(fields[k0:k0 + _BATCH], wl[k0:k0 + _BATCH], pitch, distances,
-                                S, aperture)
-                       for k0 in range(0, K, _BATCH)], dim=1)  # (D,K,S,S)
+        u = _batches([_fan_out(fields[k0:k0 + _BATCH], wl[k0:k0 + _BATCH], pitch, distances,
+                               S, aperture)
+                      for k0 in range(0, K, _BATCH)], 1)  # (D,K,S,S)
         if get_complex:
-            res = u
+            out = torch.zeros((F, D, C, S, S), dtype=torch.complex64, device=dev)
+            for k, (f, c, _) in enumerate(pairs):
+                out[f, :, c] = u[:, k]
         else:
-            res = torch.empty((D, K, S, S), dtype=torch.float32, device=dev)
+            out = torch.empty((F, D, C, S, S), dtype=torch.float32, device=dev)
             with torch.cuda.device(dev):
-                _lib.check(lib.hrf_recon_intensity(u.data_ptr(), u.numel(), res.data_ptr(),
-                                                   _lib.stream_ptr(dev)))
-        for k, (f, c, _) in enumerate(pairs):
-            out[f, :, c] = res[:, k]
+                _lib.check(lib.hrf_recon_intensity_planes(u.data_ptr(), F, D, C, hw, fr, ch, pw,
+                                                          sc, K, out.data_ptr(),
+                                                          _lib.stream_ptr(dev)))
         ctx.save_for_backward(phases, amplitude, u)
         return out
 
@@ -114,20 +120,25 @@ class _Reconstruct(torch.autograd.Function):
         dev = phases.device
         K, hw = len(pairs), S * S
         lib = _lib.load()
-        g = torch.stack([grad_out[f, :, c] for f, c, _ in pairs], dim=1).contiguous()
+        fr, ch, pw, sc = _arrays(pairs, scales)
         if get_complex:
-            gu = g.to(torch.complex64).contiguous()
+            gu = torch.stack([grad_out[f, :, c] for f, c, _ in pairs], dim=1)
+            gu = gu.to(torch.complex64).contiguous()
         else:
-            g = g.to(torch.float32).contiguous()
+            g = grad_out.to(torch.float32).resolve_neg()
+            # one stride over the pixels: rows that do not follow on are copied
+            if g.stride(3) != S * g.stride(4):
+                g = g.contiguous()
+            gs = (ctypes.c_int64 * 4)(g.stride(0), g.stride(1), g.stride(2), g.stride(4))
             gu = torch.empty_like(u)
             with torch.cuda.device(dev):
-                _lib.check(lib.hrf_recon_intensity_backward(u.data_ptr(), g.data_ptr(), u.numel(),
-                                                            gu.data_ptr(), _lib.stream_ptr(dev)))
+                _lib.check(lib.hrf_recon_intensity_planes_backward(
+                    u.data_ptr(), g.data_ptr(), gs, F, len(distances), C, hw, fr, ch, pw, sc, K,
+                    gu.data_ptr(), _lib.stream_ptr(dev)))
         wl = [wavelengths[c] for _, c, _ in pairs]
-        gfields = torch.cat([_fan_in(gu[:, k0:k0 + _BATCH].contiguous(), wl[k0:k0 + _BATCH],
-                                     pitch, distances, S, aperture)
-                             for k0 in range(0, K, _BATCH)], dim=0)
-        fr, ch, pw, sc = _arrays(pairs, scales)
+        gfields = _batches([_fan_in(gu[:, k0:k0 + _BATCH].contiguous(), wl[k0:k0 + _BATCH],
+                                    pitch, distances, S, aperture)
+                            for k0 in range(0, K, _BATCH)], 0)
         g_amp = torch.empty_like(amplitude)
         g_phase = torch.empty_like(phases)
         with torch.cuda.device(dev):

@@ -423,6 +423,25 @@ int hrf_recon_intensity(const void* field, int64_t n, float* intensity, void* st
 int hrf_recon_intensity_backward(const void* field, const float* grad_intensity, int64_t n,
                                  void* grad_field, void* stream);
 
+/* The intensities of K propagated pair fields (D, K, hw) in the result's
+ * layout: intensity (F, D, C, hw) float32, zero where (f, c) is no pair
+ * (fully overwritten; the pairs are distinct; powers and scales as above,
+ * unused). */
+int hrf_recon_intensity_planes(const void* field, int32_t F, int32_t D, int32_t C, int64_t hw,
+                               const int32_t* frames, const int32_t* channels,
+                               const float* powers, const float* scales, int32_t K,
+                               float* intensity, void* stream);
+
+/* Its backward: grad_field (D, K, hw) = 2 grad_intensity field, the gradient
+ * (F, D, C, hw) read with grad_strides[4], the elements between consecutive
+ * frames, depths, channels and pixels. */
+int hrf_recon_intensity_planes_backward(const void* field, const float* grad_intensity,
+                                        const int64_t* grad_strides, int32_t F, int32_t D,
+                                        int32_t C, int64_t hw, const int32_t* frames,
+                                        const int32_t* channels, const float* powers,
+                                        const float* scales, int32_t K, void* grad_field,
+                                        void* stream);
+
 /* Backward of hrf_recon_fields: grad_amplitude (C, hw) and grad_phase
  * (F, hw), summed over the pairs (fully overwritten). */
 int hrf_recon_fields_backward(const float* amplitude, const float* phase, int32_t F, int32_t C,

@@ -1,0 +1,121 @@
+"""The reconstruction's intensity passes that write the (frames, depths,
+channels, m, n) result and read its gradient in place: every laser-power
+pattern (some, all pairs; frames and channels without a pair), pixel counts
+with and without wide accesses, and gradients of every stride kind.
+
+The intensities are the squared complex output: two float32 products and a
+sum of non-negative terms, so within 3 ulp (4e-7 relative) of it.  Gradients
+against the oracle within 1e-4 relative L2, the reconstruction's bar; a
+gradient read in place and its contiguous copy give the same bits."""
+import numpy as np
+import pytest
+
+from conftest import rel_l2
+from test_gpu_reconstruction import PITCH, WL, _inputs, _prop
+
+pytestmark = pytest.mark.gpu
+
+POWERS = {
+    "eye": np.eye(3),
+    "one": [[0, 0, 0], [0, 0, 0.5], [0, 0, 0]],
+    "frame_off": [[0.3, 1.0, 0], [0, 0, 0], [1.2, 0.2, 0]],
+    "all": [[0.3, 1.0, 2.0], [0.4, 0.7, 1.4], [1.2, 0.2, 0.9]],
+}
+
+
+def _run(S, distances, powers, grad_of):
+    import torch
+
+    phases, amp = _inputs(S, seed=S)
+    prop = _prop(S, distances, laser_channel_power=torch.tensor(np.asarray(powers, np.float32)))
+    ph = torch.from_numpy(phases).cuda().requires_grad_(True)
+    am = torch.from_numpy(amp).cuda().requires_grad_(True)
+    out = prop.reconstruct(ph, am, no_grad=False)
+    g = grad_of(out)
+    out.backward(g)
+    with torch.no_grad():
+        z = prop.reconstruct(ph, am, get_complex=True)
+    return phases, amp, out.detach().cpu().numpy(), z.cpu().numpy(), g, ph.grad, am.grad
+
+
+@pytest.mark.parametrize("powers", list(POWERS))
+@pytest.mark.parametrize("S,distances", [(32, [1e-3, -2e-3]), (30, [1e-3]), (34, [0.0, 2e-3])])
+def test_intensity_planes(hrf, oracle_mod, S, distances, powers):
+    import torch
+
+    P = np.asarray(POWERS[powers], np.float64)
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    phases, amp, out, z, g, g_ph, g_am = _run(
+        S, distances, P, lambda o: torch.randn(o.shape, device="cuda", generator=gen))
+    print(f"S={S} D={len(distances)} powers={powers}", flush=True)
+    z = z.astype(np.complex128)
+    np.testing.assert_allclose(out, z.real ** 2 + z.imag ** 2, rtol=4e-7, atol=0)
+    e_ph, e_am = oracle_mod.reconstruct_backward(g.cpu().numpy(), phases, amp, WL, PITCH,
+                                                 distances, S, float(S), P)
+    assert rel_l2(g_ph.cpu().numpy(), e_ph) < 1e-4
+    assert rel_l2(g_am.cpu().numpy(), e_am) < 1e-4
+    for f in np.flatnonzero(~P.any(axis=1)):
+        assert not g_ph[f].any()
+    for c in np.flatnonzero(~P.any(axis=0)):
+        assert not g_am[c].any()
+
+
+@pytest.mark.parametrize("S", [32, 34])
+@pytest.mark.parametrize("kind", ["expanded", "transposed", "offset", "channels_last", "negated"])
+def test_gradient_read_in_place(hrf, S, kind):
+    import torch
+
+    def grad_of(o):
+        gen = torch.Generator(device="cuda").manual_seed(2)
+        r = lambda *s: torch.randn(*s, device="cuda", generator=gen)
+        F, D, C = o.shape[:3]
+        if kind == "expanded":
+            return r(1, 1, 1, 1, 1).expand(o.shape)
+        if kind == "transposed":
+            return r(F, D, C, S, S).transpose(3, 4)
+        if kind == "offset":  # planes that start 4 bytes off
+            return r(F * D * C * S * S + 1)[1:].view(o.shape)
+        if kind == "channels_last":
+            return r(F, D, S, S, C).permute(0, 1, 4, 2, 3)
+        return torch.complex(r(o.shape), r(o.shape)).conj().imag
+
+    a = _run(S, [1e-3, -1e-3], POWERS["frame_off"], grad_of)
+    b = _run(S, [1e-3, -1e-3], POWERS["frame_off"],
+             lambda o: grad_of(o).resolve_neg().contiguous().clone())
+    print(f"S={S} {kind}", flush=True)
+    assert torch.equal(a[5], b[5])
+    assert torch.equal(a[6], b[6])
+
+
+@pytest.mark.parametrize("hw,offset", [(1, 0), (35, 0), (1023, 0), (1024, 1), (1028, 0)])
+def test_entries_at_any_pixel_count(hrf, hw, offset):
+    """The C entries where planes or buffers do not start on 16 bytes."""
+    import ctypes
+
+    import torch
+    from complex_valued_holographic_radiance_fields_amd import _lib
+
+    F, D, C, pairs = 2, 3, 2, [(1, 0), (0, 1)]
+    K, lib = len(pairs), _lib.load()
+    fr = (ctypes.c_int32 * K)(*[f for f, _ in pairs])
+    ch = (ctypes.c_int32 * K)(*[c for _, c in pairs])
+    one = (ctypes.c_float * K)(*[1.0] * K)
+    gen = torch.Generator(device="cuda").manual_seed(hw)
+    u = torch.view_as_complex(torch.randn(D, K, hw, 2, device="cuda", generator=gen))
+    g = torch.randn(F, D, C, hw, device="cuda", generator=gen)
+    buf = torch.full((F * D * C * hw + offset,), float("nan"), device="cuda")
+    out, gu = buf[offset:].view(F, D, C, hw), torch.empty_like(u)
+    st = _lib.stream_ptr(u.device)
+    print(f"hw={hw} offset={offset}", flush=True)
+    _lib.check(lib.hrf_recon_intensity_planes(u.data_ptr(), F, D, C, hw, fr, ch, one, one, K,
+                                              out.data_ptr(), st))
+    gs = (ctypes.c_int64 * 4)(*g.stride())
+    _lib.check(lib.hrf_recon_intensity_planes_backward(u.data_ptr(), g.data_ptr(), gs, F, D, C,
+                                                       hw, fr, ch, one, one, K, gu.data_ptr(),
+                                                       st))
+    exp = torch.zeros_like(out)
+    for k, (f, c) in enumerate(pairs):
+        exp[f, :, c] = u[:, k].real.square() + u[:, k].imag.square()
+        assert torch.equal(gu[:, k], torch.complex(2 * g[f, :, c] * u[:, k].real,
+                                                   2 * g[f, :, c] * u[:, k].imag))
+    torch.testing.assert_close(out, exp, rtol=4e-7, atol=0)
