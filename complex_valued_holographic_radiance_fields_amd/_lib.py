@@ -7,6 +7,7 @@ if the library is missing or fails to load, importing the package raises.
 """
 from __future__ import annotations
 
+import contextlib
 import ctypes
 import os
 import threading
@@ -189,8 +190,23 @@ def check(status: int) -> None:
         raise RuntimeError((msg or b"hrf: unknown error").decode(errors="replace"))
 
 
+_SAME_DEVICE = contextlib.nullcontext()
+
+
+def on_device(device: torch.device):
+    """torch.cuda.device(device), or nothing to enter where that device is the
+    current one already (a switch and its return cost a small call 3 us)."""
+    if device.index == torch.cuda.current_device():
+        return _SAME_DEVICE
+    return torch.cuda.device(device)
+
+
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's handle (without a torch.cuda.Stream around it)."""
+    index = device.index
+    if index is None:
+        index = torch.cuda.current_device()
+    return torch._C._cuda_getCurrentRawStream(index)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
@@ -230,7 +246,7 @@ _WORKSPACES: dict = {}
 def workspace(purpose: str, device: torch.device, stream: int, nbytes: int) -> torch.Tensor:
     """A uint8 device buffer of at least `nbytes` bytes for `purpose` on
     (`device`, `stream`) for the calling host thread."""
-    key = (purpose, str(device), int(stream), threading.get_ident())
+    key = (purpose, device, stream, threading.get_ident())
     buf = _WORKSPACES.get(key)
     if buf is None or buf.numel() < nbytes:
         buf = torch.empty(max(int(nbytes), 1), dtype=torch.uint8, device=device)

@@ -56,7 +56,7 @@ def grad_norm_clip_coef(parameters, max_norm: float) -> tuple[torch.Tensor, torc
     lib = _lib.load()
     out = torch.empty(2, dtype=torch.float32, device=dev)
     arr, nums = _ptr_array(grads)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         stream = _lib.stream_ptr(dev)
         wbytes = lib.hrf_grad_norm_workspace_size(nums, len(grads))
         ws = _lib.workspace("grad_norm", dev, stream, wbytes)
@@ -82,7 +82,7 @@ def clip_grad_norm_(parameters, max_norm: float, norm_type: float = 2.0,
     dev = grads[0].device
     lib = _lib.load()
     arr, nums = _ptr_array(grads)
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         _lib.check(lib.hrf_scale_grads(arr, nums, len(grads), coef.data_ptr(),
                                        _lib.stream_ptr(dev)))
     return total
@@ -198,7 +198,7 @@ class Adan(Optimizer):
             cfg = _lib.HrfAdanConfig(b1, b2, b3, eps, wd, clip, int(no_prox))
             arr = (_lib.HrfAdanTensor * len(items))(*items)
             gs = grad_scale.to(dev) if grad_scale is not None else None
-            with torch.cuda.device(dev):
+            with _lib.on_device(dev):
                 _lib.check(lib.hrf_adan_step(arr, len(items), ctypes.byref(cfg), _lib.ptr(gs),
                                              _lib.stream_ptr(dev)))
         del keep

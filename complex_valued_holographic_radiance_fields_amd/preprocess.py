@@ -91,7 +91,7 @@ def forward(means, pre_act_quats, pre_act_scales, colours, pre_act_phase, pre_ac
     R, T = _camera(R, T, prm.device)
     lib = _lib.load()
     dev = prm.device
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         stream = _lib.stream_ptr(dev)
         wbytes = lib.hrf_preprocess_workspace_size(prm.n, prm.C, prm.P)
         ws = _lib.workspace("preprocess", dev, stream, wbytes)
@@ -144,7 +144,7 @@ def backward(grads, means, pre_act_quats, pre_act_scales, colours, pre_act_phase
     gin = _lib.HrfSelectedGrads(*[_lib.ptr(g) for g in gs])
     gout = _lib.HrfParamGrads(*[t.data_ptr() for t in out])
     lib = _lib.load()
-    with torch.cuda.device(prm.device):
+    with _lib.on_device(prm.device):
         stream = _lib.stream_ptr(prm.device)
         wbytes = lib.hrf_preprocess_workspace_size(prm.n, prm.C, prm.P)
         ws = _lib.workspace("preprocess", prm.device, stream, wbytes)

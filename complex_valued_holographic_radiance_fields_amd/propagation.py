@@ -43,9 +43,9 @@ def _c64(t: torch.Tensor, name: str) -> torch.Tensor:
     return t.contiguous()
 
 
-def _workspace(P: int, C: int, S: int, dev) -> tuple[torch.Tensor, int]:
+def _workspace(P: int, C: int, S: int, dev, stream: int) -> tuple[torch.Tensor, int]:
     nbytes = _lib.load().hrf_asm_workspace_size(P, C, S)
-    return _lib.workspace("asm", dev, _lib.stream_ptr(dev), nbytes), nbytes
+    return _lib.workspace("asm", dev, stream, nbytes), nbytes
 
 
 def propagate(field: torch.Tensor, wavelength, pixel_pitch, distance, size,
@@ -58,12 +58,13 @@ def propagate(field: torch.Tensor, wavelength, pixel_pitch, distance, size,
     H, W = field.shape
     out = torch.empty((S, S), dtype=torch.complex64, device=field.device)
     lib = _lib.load()
-    with torch.cuda.device(field.device):
-        ws, nb = _workspace(1, 1, S, field.device)
+    with _lib.on_device(field.device):
+        stream = _lib.stream_ptr(field.device)
+        ws, nb = _workspace(1, 1, S, field.device, stream)
         _lib.check(lib.hrf_asm_forward(field.data_ptr(), H, W, S, _as_float(wavelength),
                                        _as_float(pixel_pitch), _as_float(distance),
                                        _as_float(aperture_size), out.data_ptr(), ws.data_ptr(),
-                                       nb, _lib.stream_ptr(field.device)))
+                                       nb, stream))
     return out
 
 
@@ -77,12 +78,13 @@ def propagate_adjoint(grad_out: torch.Tensor, input_size, wavelength, pixel_pitc
     H, W = int(input_size[0]), int(input_size[1])
     out = torch.empty((H, W), dtype=torch.complex64, device=grad_out.device)
     lib = _lib.load()
-    with torch.cuda.device(grad_out.device):
-        ws, nb = _workspace(1, 1, S, grad_out.device)
+    with _lib.on_device(grad_out.device):
+        stream = _lib.stream_ptr(grad_out.device)
+        ws, nb = _workspace(1, 1, S, grad_out.device, stream)
         _lib.check(lib.hrf_asm_adjoint(grad_out.data_ptr(), H, W, S, _as_float(wavelength),
                                        _as_float(pixel_pitch), _as_float(distance),
                                        _as_float(aperture_size), out.data_ptr(), ws.data_ptr(),
-                                       nb, _lib.stream_ptr(grad_out.device)))
+                                       nb, stream))
     return out
 
 
@@ -108,12 +110,13 @@ def multiplane(fields: torch.Tensor, wavelengths, pixel_pitch, distances, size,
     S = _square_size(size)
     out = torch.empty((C, S, S), dtype=torch.complex64, device=fields.device)
     lib = _lib.load()
-    with torch.cuda.device(fields.device):
-        ws, nb = _workspace(P, C, S, fields.device)
+    with _lib.on_device(fields.device):
+        stream = _lib.stream_ptr(fields.device)
+        ws, nb = _workspace(P, C, S, fields.device, stream)
         _lib.check(lib.hrf_asm_multiplane_forward(
             fields.data_ptr(), P, C, H, W, S, _host_f32(wl), _host_f32(ds),
             _as_float(pixel_pitch), _as_float(aperture_size), out.data_ptr(), ws.data_ptr(), nb,
-            _lib.stream_ptr(fields.device)))
+            stream))
     return out
 
 
@@ -133,12 +136,13 @@ def multiplane_adjoint(grad_holo: torch.Tensor, field_hw, wavelengths, pixel_pit
                            f"got {tuple(grad_holo.shape)}")
     out = torch.empty((P, C, H, W), dtype=torch.complex64, device=grad_holo.device)
     lib = _lib.load()
-    with torch.cuda.device(grad_holo.device):
-        ws, nb = _workspace(P, C, S, grad_holo.device)
+    with _lib.on_device(grad_holo.device):
+        stream = _lib.stream_ptr(grad_holo.device)
+        ws, nb = _workspace(P, C, S, grad_holo.device, stream)
         _lib.check(lib.hrf_asm_multiplane_adjoint(
             grad_holo.data_ptr(), P, C, H, W, S, _host_f32(wl), _host_f32(ds),
             _as_float(pixel_pitch), _as_float(aperture_size), out.data_ptr(), ws.data_ptr(), nb,
-            _lib.stream_ptr(grad_holo.device)))
+            stream))
     return out
 
 
@@ -180,7 +184,7 @@ def multidistance(fields: torch.Tensor, wavelengths, pixel_pitch, distances, siz
     S = _square_size(size)
     out = torch.empty((len(ds), C, S, S), dtype=torch.complex64, device=fields.device)
     lib = _lib.load()
-    with torch.cuda.device(fields.device):
+    with _lib.on_device(fields.device):
         ws, nb = _md_workspace(len(ds), C, S, fields.device)
         _lib.check(lib.hrf_asm_multidistance_forward(
             fields.data_ptr(), len(ds), C, H, W, S, _host_f32(wl), _host_f32(ds),
@@ -203,7 +207,7 @@ def multidistance_adjoint(grad_out: torch.Tensor, field_hw, wavelengths, pixel_p
                            f"got {tuple(grad_out.shape)}")
     out = torch.empty((C, H, W), dtype=torch.complex64, device=grad_out.device)
     lib = _lib.load()
-    with torch.cuda.device(grad_out.device):
+    with _lib.on_device(grad_out.device):
         ws, nb = _md_workspace(D, C, S, grad_out.device)
         _lib.check(lib.hrf_asm_multidistance_adjoint(
             grad_out.data_ptr(), D, C, H, W, S, _host_f32(wl), _host_f32(ds),
@@ -244,7 +248,7 @@ def _spectral(args, adjoint: bool):
     out_re = torch.zeros_like(ts[0])
     out_im = torch.zeros_like(ts[0])
     lib = _lib.load()
-    with torch.cuda.device(ts[0].device):
+    with _lib.on_device(ts[0].device):
         s = _lib.stream_ptr(ts[0].device)
         if adjoint:
             fr = f_re.contiguous()

@@ -22,7 +22,7 @@ def _f32c(t: torch.Tensor, name: str, shape_tail: Tuple[int, ...] | None = None)
         raise RuntimeError(f"{name} must be a GPU tensor (the HIP rasterizer has no CPU path)")
     if t.dtype != torch.float32:
         raise RuntimeError(f"{name} must be float32 (got {t.dtype})")
-    if shape_tail is not None and tuple(t.shape[1:]) != shape_tail:
+    if shape_tail is not None and t.shape[1:] != shape_tail:
         raise RuntimeError(f"{name} must have shape (N, {', '.join(map(str, shape_tail))}), "
                            f"got {tuple(t.shape)}")
     return t.contiguous()
@@ -122,7 +122,7 @@ def forward(cam_means_3D, z_vals, quats, scales, colours, phase, opacities, plan
     lib = _lib.load()
     dev = inp.device
     P, C, H, W = inp.P, inp.C, inp.H, inp.W
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         stream = _lib.stream_ptr(dev)
         gbytes = lib.hrf_raster_geom_workspace_size(inp.n, C, P)
         if keep_geometry:
@@ -135,7 +135,7 @@ def forward(cam_means_3D, z_vals, quats, scales, colours, phase, opacities, plan
         final_T = torch.empty((P, H, W), dtype=torch.float32, device=dev)
         n_contrib = torch.empty((P, H, W), dtype=torch.int32, device=dev)
         ranges = torch.empty((inp.ntiles, 2), dtype=torch.int32, device=dev)
-        key = (str(dev), W, H, P, inp.n)
+        key = (dev, W, H, P, inp.n)
         last = _LAST_PAIRS.get(key, 0)
         cap = last + last // 8 + 4096 if last > 0 else 0
         if cap > 0:
@@ -208,7 +208,7 @@ def backward_prepare(cam_means_3D, z_vals, quats, scales, colours, phase, opacit
     n, C, P = inp.n, inp.C, inp.P
     if n == 0:
         return
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         # the workspace the backward on the current stream will use
         wbytes = lib.hrf_raster_backward_workspace_size(n, C, P)
         ws = _lib.workspace("raster_bwd", dev, _lib.stream_ptr(dev), wbytes)
@@ -265,7 +265,7 @@ def backward(grad_output, cam_means_3D, z_vals, quats, scales, colours, phase, o
     g_pl = torch.empty((n, P), **opts)
     if n == 0:
         return [g_cam, g_z, g_q, g_s, g_col, g_ph, g_o, g_pl]
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         stream = _lib.stream_ptr(dev)
         wbytes = lib.hrf_raster_backward_workspace_size(n, C, P)
         ws = _lib.workspace("raster_bwd", dev, stream, wbytes)

@@ -88,7 +88,7 @@ class _Reconstruct(torch.autograd.Function):
         fr, ch, pw, sc = _arrays(pairs, scales)
         lib = _lib.load()
         fields = torch.empty((K, S, S), dtype=torch.complex64, device=dev)
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             stream = _lib.stream_ptr(dev)
             _lib.check(lib.hrf_recon_fields(amplitude.data_ptr(), phases.data_ptr(), F, C, hw,
                                             fr, ch, pw, sc, K, fields.data_ptr(), stream))
@@ -102,7 +102,7 @@ class _Reconstruct(torch.autograd.Function):
                 out[f, :, c] = u[:, k]
         else:
             out = torch.empty((F, D, C, S, S), dtype=torch.float32, device=dev)
-            with torch.cuda.device(dev):
+            with _lib.on_device(dev):
                 _lib.check(lib.hrf_recon_intensity_planes(u.data_ptr(), F, D, C, hw, fr, ch, pw,
                                                           sc, K, out.data_ptr(),
                                                           _lib.stream_ptr(dev)))
@@ -131,7 +131,7 @@ class _Reconstruct(torch.autograd.Function):
                 g = g.contiguous()
             gs = (ctypes.c_int64 * 4)(g.stride(0), g.stride(1), g.stride(2), g.stride(4))
             gu = torch.empty_like(u)
-            with torch.cuda.device(dev):
+            with _lib.on_device(dev):
                 _lib.check(lib.hrf_recon_intensity_planes_backward(
                     u.data_ptr(), g.data_ptr(), gs, F, len(distances), C, hw, fr, ch, pw, sc, K,
                     gu.data_ptr(), _lib.stream_ptr(dev)))
@@ -141,7 +141,7 @@ class _Reconstruct(torch.autograd.Function):
                             for k0 in range(0, K, _BATCH)], 0)
         g_amp = torch.empty_like(amplitude)
         g_phase = torch.empty_like(phases)
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             _lib.check(lib.hrf_recon_fields_backward(
                 amplitude.data_ptr(), phases.data_ptr(), F, C, hw, fr, ch, pw, sc, K,
                 gfields.data_ptr(), g_amp.data_ptr(), g_phase.data_ptr(), _lib.stream_ptr(dev)))
