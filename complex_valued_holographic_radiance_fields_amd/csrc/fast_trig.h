@@ -40,4 +40,34 @@ __device__ __forceinline__ void sincos_big_ff(float x, float* s, float* c) {
   *c = __builtin_amdgcn_cosf(rev);
 }
 
+// The same reduction down to a quadrant, and polynomials instead of the
+// hardware functions: with rev = q / 4 + f, |f| <= 1/8, the remainder keeps
+// two more bits than a half revolution does, and sin(2 pi f) = f S(f^2),
+// cos(2 pi f) = 1 + f^2 C(f^2) with cubic S and C (interpolated at Chebyshev
+// nodes of f^2 in [0, 1/64], rounded to float).  2.1e-8 rms off float64 in
+// each, where the hardware functions of a rounded half revolution leave about
+// 6e-8: for the transforms that replace ones whose transfer function called
+// sincosf (1.5e-8).
+__device__ __forceinline__ void sincos_big_quad(float x, float* s, float* c) {
+  constexpr float kHi = 0.15915493667125701904f;
+  constexpr float kLo = 6.4206383167313347657e-09f;
+  const float hi = x * kHi;
+  const float lo = fmaf(x, kLo, fmaf(x, kHi, -hi));
+  const float r = hi - __builtin_rintf(hi);       // exact, in [-0.5, 0.5]
+  const float q4 = __builtin_rintf(4.0f * r);     // -2 .. 2
+  const float f = fmaf(q4, -0.25f, r) + lo;       // the fma is exact
+  const float g = f * f;
+  const float sn =
+      f * fmaf(g, fmaf(g, fmaf(g, -75.40184020996094f, 81.59254455566406f), -41.3416633605957f),
+               6.2831854820251465f);
+  const float cs =
+      fmaf(g, fmaf(g, fmaf(g, fmaf(g, 59.42423629760742f, -85.44882202148438f),
+                           64.93936920166016f), -19.739208221435547f), 1.0f);
+  const int q = static_cast<int>(q4);
+  const float a = (q & 1) ? cs : sn, b = (q & 1) ? sn : cs;
+  // quadrants 2, 3 negate the sine, 1, 2 the cosine (q mod 4)
+  *s = (q & 2) ? -a : a;
+  *c = ((q + 1) & 2) ? -b : b;
+}
+
 }  // namespace hrf

@@ -33,6 +33,10 @@ __global__ void k_sincos(const float* x, float* s, float* c, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) hrf::sincos_big(x[i], s + i, c + i);
 }
+__global__ void k_sincos_quad(const float* x, float* s, float* c, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) hrf::sincos_big_quad(x[i], s + i, c + i);
+}
 
 // Calibration kernels of known VALU work, for reading the SQ counters
 // (SQ_INSTS_VALU, SQ_ACTIVE_INST_VALU, SQ_INSTS_VALU_TRANS_F32) against a
@@ -179,6 +183,11 @@ extern "C" int calib_valu_exp(float* out, int blocks, int iters, float a, void* 
 
 extern "C" int trig_test_sincos(const float* x, float* s, float* c, int n) {
   hipLaunchKernelGGL(k_sincos, dim3((n + 255) / 256), dim3(256), 0, nullptr, x, s, c, n);
+  return static_cast<int>(hipDeviceSynchronize());
+}
+
+extern "C" int trig_test_sincos_quad(const float* x, float* s, float* c, int n) {
+  hipLaunchKernelGGL(k_sincos_quad, dim3((n + 255) / 256), dim3(256), 0, nullptr, x, s, c, n);
   return static_cast<int>(hipDeviceSynchronize());
 }
 
