@@ -15,6 +15,8 @@
 //   9   (556 x 742)   1484   1195 / 1143 us       390 / 340 us   (chirp)
 //   3   (1424 x 1900) 3800   3000 / 2945 us       839 / 791 us   (chirp)
 //
+// (with the hardware sine and cosine in the transfer function; turn_quad adds
+// 2-8% to a pass pair).
 // The column passes are bound by VALU issue and the latency between their
 // barriers (1008 points, 18 fields: 66 us of the 101), the row passes by
 // memory latency.

@@ -249,11 +249,14 @@ int hrf_asm_spectral_backward(const float* grad_re, const float* grad_im,
                               float pixel_pitch, void* stream);
 
 /* Workspace for the whole-propagation entry points below: M = 2*S.
- * Grids with M in {128, 160, 192, 512, 1024, 1600, 2016, 2048} run the
- * fused hand-written LDS-FFT kernels (row pass with the zero pad, column
- * pass with the transfer-function multiply summed over planes and the row
- * crop, inverse row pass with the column crop and 1/M^2); other even sizes
- * run the same arithmetic around hipFFT transforms. */
+ * Every M that is a multiple of 4 in 32..4096 runs the fused hand-written
+ * LDS-FFT kernels (row pass with the zero pad, column pass with the
+ * transfer-function multiply summed over planes and the row crop, inverse
+ * row pass with the column crop and 1/M^2): compiled plans for 128, 160, 192,
+ * 512, 1024, 1600, 2016, 2048, 3840 and 4096, run-time radices for the other
+ * lengths with factors 2, 3, 5 and 7, a chirp transform for the rest (fields
+ * of at most half the grid).  Larger or smaller M, and wider fields on a chirp
+ * length, run the same arithmetic around hipFFT transforms. */
 size_t hrf_asm_workspace_size(int32_t planes, int32_t channels, int32_t size);
 
 /* One field (H,W) c64 -> (S,S) c64: centred zero pad to (2S,2S), FFT,
