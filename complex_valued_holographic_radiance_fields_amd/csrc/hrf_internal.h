@@ -221,8 +221,6 @@ struct GeomBwdParams {
 };
 int launch_geom_backward(const GeomBwdParams& p, hipStream_t s);
 
-// Scan scratch sizing (block-sum pyramid of an n-element scan).
-
 // Stable LSD radix sort of (u32 key, u32 value) pairs over bits
 // [0, end_bit).  Ping-pongs between (ka,va) and (kb,vb); returns in
 // *result_in_b whether the sorted data ended in (kb,vb).  With run_flag, the
